@@ -242,9 +242,14 @@ static void launch_pass_t(const DevView& v, int mode, int iteration, int parity,
     const int tiles_x = (v.Wc + kTX - 1) / kTX;
     const int tiles = tiles_x * ((v.H + kTY - 1) / kTY);
     const dim3 grid(((tiles + 7) / 8) * 8);
+    // LDS the kernel does not use, to hold fewer workgroups on a CU: the 121-tap
+    // initial cost, whose random hypotheses scatter the gathers, thrashes the L1
+    // with the 5 waves to a SIMD that its registers allow (1600x1200, 4 sources,
+    // FP32: 0.48 ms a colour, 0.44 with 3.5; FP16's halved lines: no difference)
+    constexpr unsigned kIdleLds = NT >= 11 && STORE == kStoreF32 ? 6144 : 0;
     if (mode == kPassCost)
-        hipLaunchKernelGGL((pm_cost_kernel<NT, ST, STORE, kTX, kTY>), grid, dim3(kTX * kTY), 0, st,
-                           v, parity, tiles_x, tiles);
+        hipLaunchKernelGGL((pm_cost_kernel<NT, ST, STORE, kTX, kTY>), grid, dim3(kTX * kTY),
+                           kIdleLds, st, v, parity, tiles_x, tiles);
     else
         hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY>), grid, dim3(kTX * kTY), 0,
                            st, v, iteration, parity, pass_seed, tiles_x, tiles);

@@ -220,29 +220,37 @@ template <> struct StateIO<true> {
 // plane; an invalid tap's index goes nowhere and reads zeros.
 template <int STORE> struct SrcImage;
 template <> struct SrcImage<kStoreF32> {
+    typedef float4 Quad;
     __amdgpu_buffer_rsrc_t rsrc;
     unsigned pitch;
     __device__ SrcImage(const DevView& v, int s)
         : rsrc(make_rsrc(v.src_coef[s], v.coef_bytes / 8, 8)), pitch((unsigned)v.pitch_plain) {}
-    __device__ __forceinline__ float sample(int ix, int iy, float au, float aw, bool ok = true) const
+    __device__ __forceinline__ Quad load(int ix, int iy, bool ok = true) const
     {
         unsigned idx = __umul24((unsigned)iy, pitch) + (unsigned)ix;
         idx = ok ? idx : kIdxNowhere;
-        const float4 q = __builtin_bit_cast(float4, struct_load_b128(rsrc, (int)idx, 0, 0, 0));
+        return __builtin_bit_cast(float4, struct_load_b128(rsrc, (int)idx, 0, 0, 0));
+    }
+    static __device__ __forceinline__ float lerp(const Quad& q, float au, float aw)
+    {
         const float c0 = fmaf(aw, q.y, q.x), c1 = fmaf(aw, q.w, q.z);
         return fmaf(au, c1 - c0, c0);
     }
 };
 template <> struct SrcImage<kStoreF16> {
+    typedef half4_t Quad;
     __amdgpu_buffer_rsrc_t rsrc;
     unsigned pitch;
     __device__ SrcImage(const DevView& v, int s)
         : rsrc(make_rsrc(v.src_coef[s], v.coef_bytes / 4, 4)), pitch((unsigned)v.pitch_plain) {}
-    __device__ __forceinline__ float sample(int ix, int iy, float au, float aw, bool ok = true) const
+    __device__ __forceinline__ Quad load(int ix, int iy, bool ok = true) const
     {
         unsigned idx = __umul24((unsigned)iy, pitch) + (unsigned)ix;
         idx = ok ? idx : kIdxNowhere;
-        const half4_t q = __builtin_bit_cast(half4_t, struct_load_b64(rsrc, (int)idx, 0, 0, 0));
+        return __builtin_bit_cast(half4_t, struct_load_b64(rsrc, (int)idx, 0, 0, 0));
+    }
+    static __device__ __forceinline__ float lerp(const Quad& q, float au, float aw)
+    {
         const float c0 = fmaf(aw, (float)q.y, (float)q.x), c1 = fmaf(aw, (float)q.w, (float)q.z);
         return fmaf(au, c1 - c0, c0);
     }
@@ -288,6 +296,20 @@ __device__ __forceinline__ WinRef window_ref_sums(const float* __restrict__ lwin
     return WinRef{sr, srr};
 }
 
+// Taps of a window row whose gathers are in flight together (C of tap_window).
+// Half-pass: rows of up to 7 taps whole, 9 and 11 taps as 5 + 4 and 6 + 5.  With
+// two whole rows of 11 in flight (as many gathers as the compiler would keep
+// registers for) that kernel held 167 registers and 3 waves to a SIMD, its
+// unrolled loops filled more than the 64 KiB instruction cache, and a change
+// anywhere else could make it wait for each gather by itself (+23 % time); in
+// chunks it holds 119, 4 waves, and every loop is one row long: 1280x960 with 8
+// sources at stride 1, FP32, 2.00 -> 1.94 ms a half-pass.
+// Initial cost: whole rows.  Its random hypotheses scatter the gathers, the
+// L1's line rate bounds it, and chunks only add to its waits (1600x1200, 11x11
+// taps, FP32: 0.48 against 0.51 ms a colour).
+template <int NT> constexpr int kPassChunk = NT <= 7 ? NT : (NT + 1) / 2;
+template <int NT> constexpr int kCostChunk = NT;
+
 // The window's taps for one candidate and source (patchmatch_mvs.cu:273-307).
 // MASKED = false is used only when every tap is known to be inside the image;
 // it takes the reference sums from wr, which window_ref_sums forms with the
@@ -311,7 +333,7 @@ __device__ __forceinline__ WinRef window_ref_sums(const float* __restrict__ lwin
 // (cx, cy) and the columns (h00, h10), (h01, h11) may be relative to an
 // integer base (bu, bv): the taps' coordinates are then u - bu and v - bv,
 // and the base is added back to the texel index.
-template <int NT, int ST, int STORE, bool MASKED, bool ZCHK = true, int RU = (NT >= 9 ? 2 : 1)>
+template <int NT, int ST, int STORE, bool MASKED, bool ZCHK, int C>
 __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
                                            const float* __restrict__ lwin, int lp, float cx,
                                            float cy, float cz, float h00, float h01, float h10,
@@ -325,12 +347,7 @@ __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
     float s0 = 0.f;     // the shift: first valid sample of the window
     bool have = false;  // (masked loop) a valid tap has been seen
     int cnt = 0;
-    // window rows (RU at a time): by default two for the 11-tap (stride 1)
-    // rows of the half-pass, where the extra loads in flight pay, one for the
-    // 6-tap rows, where unrolling measured slower; the initial-cost pass takes
-    // its 11-tap rows one at a time too (its random hypotheses scatter the
-    // gathers: 0.751 -> 0.442 ms per colour with FP32 storage at 1600x1200)
-#pragma unroll RU
+#pragma unroll 1
     for (int jr = 0; jr < NT; ++jr) {
         const int j = jr + F < NT ? jr + F : jr + F - NT;
         const float oy = (float)(j * ST - R);
@@ -339,44 +356,62 @@ __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
         const float bz = fmaf(h21, oy, cz);
         const float* lrow = lwin + j * ST * lp;
 #pragma unroll
-        for (int ir = 0; ir < NT; ++ir) {
-            const int i = ir + F < NT ? ir + F : ir + F - NT;
-            const float ox = (float)(i * ST - R);
-            const float wx = fmaf(h00, ox, bx);
-            const float wy = fmaf(h10, ox, by);
-            const float wz = fmaf(h20, ox, bz);
-            const float rw = __builtin_amdgcn_rcpf(wz);
-            const float u = wx * rw, w = wy * rw;
-            // (a wrapped sum lands far outside [0, umax], as any invalid tap)
-            const int ix = (int)((unsigned)bu + (unsigned)cvt_flr(u));
-            const int iy = (int)((unsigned)bv + (unsigned)cvt_flr(w));
-            const float au = __builtin_amdgcn_fractf(u), aw = __builtin_amdgcn_fractf(w);
-            // |w_z| guard and 0 <= u < W-1, 0 <= v < H-1 (:289-295); an
-            // invalid tap's load goes nowhere and reads zeros (so sval = 0)
-            const bool ok = !MASKED || ((!ZCHK || fabsf(wz) >= 1e-8f) & ((unsigned)ix <= umax) &
-                                        ((unsigned)iy <= vmax));
-            const float sraw = img.sample(ix, iy, au, aw, ok);
-            float r = lrow[i * ST];
-            float sval;
-            if (MASKED) {
-                // an invalid tap read zeros; before the first valid tap s0
-                // stays 0, at it s0 becomes that tap's sample
-                s0 = have ? s0 : sraw;
-                have = have || ok;
-                sval = ok ? sraw - s0 : 0.0f;
-                r = ok ? r : 0.0f;
-                cnt += ok ? 1 : 0;
-            } else {
-                if (ir == 0) s0 = jr == 0 ? sraw : s0;
-                sval = sraw - s0;
+        for (int i0 = 0; i0 < NT; i0 += C) {
+            typename SrcImage<STORE>::Quad q[C];
+            float au[C], aw[C], rv[C];
+            bool okv[C];
+#pragma unroll
+            for (int t = 0; t < C; ++t) {
+                const int ir = i0 + t;
+                if (ir >= NT) break;
+                const int i = ir + F < NT ? ir + F : ir + F - NT;
+                const float ox = (float)(i * ST - R);
+                const float wx = fmaf(h00, ox, bx);
+                const float wy = fmaf(h10, ox, by);
+                const float wz = fmaf(h20, ox, bz);
+                const float rw = __builtin_amdgcn_rcpf(wz);
+                const float u = wx * rw, w = wy * rw;
+                // (a wrapped sum lands far outside [0, umax], as any invalid tap)
+                const int ix = (int)((unsigned)bu + (unsigned)cvt_flr(u));
+                const int iy = (int)((unsigned)bv + (unsigned)cvt_flr(w));
+                au[t] = __builtin_amdgcn_fractf(u);
+                aw[t] = __builtin_amdgcn_fractf(w);
+                // |w_z| guard and 0 <= u < W-1, 0 <= v < H-1 (:289-295); an
+                // invalid tap's load goes nowhere and reads zeros (so sval = 0)
+                okv[t] = !MASKED || ((!ZCHK || fabsf(wz) >= 1e-8f) & ((unsigned)ix <= umax) &
+                                     ((unsigned)iy <= vmax));
+                q[t] = img.load(ix, iy, okv[t]);
+                rv[t] = lrow[i * ST];
             }
-            if (MASKED) {
-                sr += r;
-                srr = fmaf(r, r, srr);
+#pragma unroll
+            for (int t = 0; t < C; ++t) {
+                const int ir = i0 + t;
+                if (ir >= NT) break;
+                const bool ok = okv[t];
+                const float sraw = SrcImage<STORE>::lerp(q[t], au[t], aw[t]);
+                float r = rv[t];
+                float sval;
+                if (MASKED) {
+                    // an invalid tap read zeros; before the first valid tap s0
+                    // stays 0, at it s0 becomes that tap's sample
+                    s0 = have ? s0 : sraw;
+                    have = have || ok;
+                    sval = ok ? sraw - s0 : 0.0f;
+                    r = ok ? r : 0.0f;
+                    cnt += ok ? 1 : 0;
+                } else {
+                    if (ir == 0) s0 = jr == 0 ? sraw : s0;
+                    sval = sraw - s0;
+                }
+                if (MASKED) {
+                    sr += r;
+                    srr = fmaf(r, r, srr);
+                }
+                ss += sval;
+                sss = fmaf(sval, sval, sss);
+                srs = fmaf(r, sval, srs);
             }
-            ss += sval;
-            sss = fmaf(sval, sval, sss);
-            srs = fmaf(r, sval, srs);
+            __builtin_amdgcn_sched_barrier(0);   // no row's loads before the last row's samples
         }
     }
     m.sr = MASKED ? sr : wr.sr;
@@ -420,6 +455,38 @@ __device__ __forceinline__ bool window_inside(float cx, float cy, float cz, floa
            (fmaf(kE, fmaf(Hq, Tz, Ty), gy) < 0.0f);
 }
 
+// True if every tap of the window provably misses the image, in front of the
+// camera and more than a pixel to one side: all u < -1, or all u > W, or the
+// same for v and H.  The extremes over the window are affine, as in
+// window_inside.  Besides the pixel, each bound is tightened by 2^-21 of
+// T_x + (W + 2^17) T_z, which covers the rounding of a tap's coordinate also
+// relative to an integer base of up to 2^17 (small windows), and u is compared
+// at W (1 + 2^-16), which covers its relative rounding at planes of 2^24
+// columns.  NaN or infinite inputs fail every comparison.
+constexpr float kOutsideBase = 131072.0f;   // 2^17
+__device__ __forceinline__ bool window_outside(float cx, float cy, float cz, float h00, float h01,
+                                               float h10, float h11, float h20, float h21, float R,
+                                               float W, float H)
+{
+    constexpr float kE = 4.76837158203125e-07f;         // 2^-21
+    constexpr float kOut = 1.0000152587890625f;         // 1 + 2^-16
+    const float Wo = fmaf(W, kOut, 1.0f), Ho = fmaf(H, kOut, 1.0f);
+    const float Tx = fmaf(R, fabsf(h00) + fabsf(h01), fabsf(cx));
+    const float Ty = fmaf(R, fabsf(h10) + fabsf(h11), fabsf(cy));
+    const float az = fabsf(h20) + fabsf(h21), Tz = fmaf(R, az, fabsf(cz));
+    const float mx = kE * fmaf(Wo + kOutsideBase, Tz, Tx);
+    const float my = kE * fmaf(Ho + kOutsideBase, Tz, Ty);
+    // maxima of w_x + w_z and w_y + w_z; minima of w_x - Wo w_z, w_y - Ho w_z
+    const float lx = fmaf(R, fabsf(h00 + h20) + fabsf(h01 + h21), cx + cz);
+    const float ly = fmaf(R, fabsf(h10 + h20) + fabsf(h11 + h21), cy + cz);
+    const float gx = fmaf(-R, fabsf(fmaf(-Wo, h20, h00)) + fabsf(fmaf(-Wo, h21, h01)),
+                          fmaf(-Wo, cz, cx));
+    const float gy = fmaf(-R, fabsf(fmaf(-Ho, h20, h10)) + fabsf(fmaf(-Ho, h21, h11)),
+                          fmaf(-Ho, cz, cy));
+    return fmaf(-kE, Tz, fmaf(-R, az, cz)) >= 1e-8f &&
+           (lx + mx < 0.0f || ly + my < 0.0f || gx - mx > 0.0f || gy - my > 0.0f);
+}
+
 // True if every tap of the window has |w_z| >= 1e-8 in its FP32 evaluation:
 // w_z is affine in the offset, so its extremes over |ox|, |oy| <= R are
 // c_z -/+ R (|h20| + |h21|), each bound tightened by 2^-21 of the terms'
@@ -444,126 +511,177 @@ __device__ __forceinline__ bool z_clear(float cz, float h20, float h21, float R)
 // in FP32 with |dx|, |dy| <= 5, so the coordinates are accurate to the FP32
 // representation of w even for grazing planes.
 // ---------------------------------------------------------------------------
-template <int NT, int ST, int STORE, int RU = (NT >= 9 ? 2 : 1)>
+// The candidate's part of the homography: g, and g.p at the window centre.
+struct CandPlane {
+    double g0, g1, g2, gc;
+};
+
+// False where n.P is too small to divide by: the candidate's cost is 2.
+__device__ __forceinline__ bool cand_plane(const DevView& v, int x, int y, double rx, double ry,
+                                           double rz, float d, float nx, float ny, float nz,
+                                           CandPlane& g)
+{
+    const double dd = d, dnx = nx, dny = ny, dnz = nz;
+    const double nP = dd * fma(dnx, rx, fma(dny, ry, dnz * rz));
+    if (fabs(nP) < 1e-8) return false;
+    const double inv = 1.0 / nP;
+    const double* ki = v.kinv_d;
+    // g = K^-T n / (n.P): the reference's factor(p) = g.p
+    g.g0 = fma(ki[0], dnx, fma(ki[3], dny, ki[6] * dnz)) * inv;
+    g.g1 = fma(ki[1], dnx, fma(ki[4], dny, ki[7] * dnz)) * inv;
+    g.g2 = fma(ki[2], dnx, fma(ki[5], dny, ki[8] * dnz)) * inv;
+    const double X = x, Y = y;
+    g.gc = fma(g.g0, X, fma(g.g1, Y, g.g2));   // factor at the window centre
+    return true;
+}
+
+// Cost 1 - NCC of one candidate plane against source s.
+template <int NT, int ST, int STORE, int C>
+__device__ __forceinline__ float source_cost(const DevView& v, int s,
+                                             const float* __restrict__ lwin, int lp,
+                                             const WinRef& wr, int x, int y, const CandPlane& g)
+{
+    constexpr int R = (NT - 1) * ST / 2;
+    constexpr int kMinCount = (NT * NT) / 2;
+    constexpr bool kLocalCoords = NT * NT <= HP3D_LOCAL_TAPS;
+    const double g0 = g.g0, g1 = g.g1, gc = g.gc;
+    const double X = x, Y = y;
+    const unsigned umax = (unsigned)(v.W - 2), vmax = (unsigned)(v.H - 2);
+    constexpr float kShrink = 0.99999904632568359375f;   // 1 - 2^-20
+    const float Wq = (float)(v.W - 1) * kShrink, Hq = (float)(v.H - 1) * kShrink;
+    const double* A = v.src[s].A;
+    const double* b = v.src[s].b;
+    // centre of the window and the two tap-step columns of H
+    const float cx = (float)fma(b[0], gc, fma(A[0], X, fma(A[1], Y, A[2])));
+    const float cy = (float)fma(b[1], gc, fma(A[3], X, fma(A[4], Y, A[5])));
+    const float cz = (float)fma(b[2], gc, fma(A[6], X, fma(A[7], Y, A[8])));
+    const float h00 = (float)fma(b[0], g0, A[0]), h01 = (float)fma(b[0], g1, A[1]);
+    const float h10 = (float)fma(b[1], g0, A[3]), h11 = (float)fma(b[1], g1, A[4]);
+    const float h20 = (float)fma(b[2], g0, A[6]), h21 = (float)fma(b[2], g1, A[7]);
+    const SrcImage<STORE> img(v, s);
+
+    // Small windows' taps relative to an integer base (bu, bv) near the
+    // centre's source position: the base comes out of the centre and the
+    // columns in FP64 (u - bu = (w_x - bu w_z) / w_z, still affine in the
+    // tap offset over w_z), so the taps' FP32 arithmetic works on u - bu,
+    // a few pixels, and rounds to ~ulp(R) instead of ~ulp(u) (1e-5 px at
+    // u ~ 100), an error a 3x3 window's NCC amplifies past 1e-4 of cost.
+    // A centre that projects beyond 2^22 pixels keeps the base 0.
+    float tx = cx, ty = cy, t00 = h00, t01 = h01, t10 = h10, t11 = h11;
+    int bu = 0, bv = 0;
+    if constexpr (kLocalCoords) {
+        const float rc = __builtin_amdgcn_rcpf(cz);
+        const float pu = cx * rc, pv = cy * rc;
+        bu = fabsf(pu) < 4194304.0f ? (int)rintf(pu) : 0;
+        bv = fabsf(pv) < 4194304.0f ? (int)rintf(pv) : 0;
+        const double nu = -(double)bu, nv = -(double)bv;
+        const double CZ = fma(b[2], gc, fma(A[6], X, fma(A[7], Y, A[8])));
+        const double H20 = fma(b[2], g0, A[6]), H21 = fma(b[2], g1, A[7]);
+        tx = (float)fma(nu, CZ, fma(b[0], gc, fma(A[0], X, fma(A[1], Y, A[2]))));
+        t00 = (float)fma(nu, H20, fma(b[0], g0, A[0]));
+        t01 = (float)fma(nu, H21, fma(b[0], g1, A[1]));
+        ty = (float)fma(nv, CZ, fma(b[1], gc, fma(A[3], X, fma(A[4], Y, A[5]))));
+        t10 = (float)fma(nv, H20, fma(b[1], g0, A[3]));
+        t11 = (float)fma(nv, H21, fma(b[1], g1, A[4]));
+    }
+
+    // The unmasked tap loop when every lane's window is inside the
+    // source image (windows with w_z < 0 throughout take the masked
+    // loop, which gives the same result).
+    const bool inside = window_inside(cx, cy, cz, h00, h01, h10, h11, h20, h21, (float)R,
+                                      Wq, Hq);
+    TapSums m;
+    // No tap of any lane's window in the image: the cost is that of no sample.
+    // (9 % of the wave evaluations of a 4-source 30-degree arc, image-edge
+    // bands that the outer sources do not see, otherwise run the masked loop
+    // for nothing.)
+    if (!__all(inside)) {
+        bool outside = window_outside(cx, cy, cz, h00, h01, h10, h11, h20, h21, (float)R,
+                                      (float)v.W, (float)v.H);
+        if constexpr (kLocalCoords)
+            outside = outside && fabsf((float)bu) <= kOutsideBase && fabsf((float)bv) <= kOutsideBase;
+        if (__all(outside)) return 2.0f;
+    }
+    if (__all(inside)) {
+        tap_window<NT, ST, STORE, false, true, C>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
+                                                   t11, h20, h21, umax, vmax, wr, m, bu, bv);
+    } else if (STORE == kStoreF16 && __all(z_clear(cz, h20, h21, (float)R))) {
+        // FP16 storage only: a third loop without the per-tap |w_z| test
+        // measured +2 % there and -12 % with FP32 storage at stride 1
+        tap_window<NT, ST, STORE, true, false, C>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
+                                                   t11, h20, h21, umax, vmax, wr, m, bu, bv);
+    } else {
+        tap_window<NT, ST, STORE, true, true, C>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
+                                                  t11, h20, h21, umax, vmax, wr, m, bu, bv);
+    }
+    const int cnt = m.cnt;
+    const float sr = m.sr, ss = m.ss, srr = m.srr, sss = m.sss, srs = m.srs;
+    float c = 2.0f;
+    if (cnt >= kMinCount) {
+        // the products of two floats are exact in FP64, so each difference
+        // rounds once with or without the FMA
+        const double fc = (double)cnt;
+        const double num = fma(fc, (double)srs, -((double)sr * (double)ss));
+        const double dr = fma(fc, (double)srr, -((double)sr * (double)sr));
+        const double ds = fma(fc, (double)sss, -((double)ss * (double)ss));
+        if (!(dr < (double)v.den_eps) && !(ds < (double)v.den_eps)) {
+            // dr, ds >= den_eps (~0.065): far from the denormal range,
+            // where rsqrtf would first rescale, so the bare v_rsq_f32
+            float ncc = (float)num * __builtin_amdgcn_rsqf((float)dr * (float)ds);
+            ncc = fmaxf(-1.0f, fminf(1.0f, ncc));
+            c = 1.0f - ncc;
+        }
+    }
+    return c;
+}
+
+// The ascending list of a candidate's smallest source costs: 3 entries
+// suffice when at most 3 are averaged (the reference's top-3), else 8.
+struct TopCosts {
+    float top[kMaxTopK];
+    __device__ __forceinline__ TopCosts()
+    {
+#pragma unroll
+        for (int k = 0; k < kMaxTopK; ++k) top[k] = 2.0f;
+    }
+    // entry k becomes the median of c and its old neighbours k - 1 and k: c if
+    // it falls between them, the lower one if c pushes it up, else unchanged
+    __device__ __forceinline__ void insert(float c, bool small_k)
+    {
+        if (small_k) {
+#pragma unroll
+            for (int k = 2; k > 0; --k) top[k] = __builtin_amdgcn_fmed3f(c, top[k - 1], top[k]);
+        } else {
+#pragma unroll
+            for (int k = kMaxTopK - 1; k > 0; --k)
+                top[k] = __builtin_amdgcn_fmed3f(c, top[k - 1], top[k]);
+        }
+        top[0] = fminf(c, top[0]);
+    }
+    __device__ __forceinline__ float mean(const DevView& v) const
+    {
+        const int k = v.top_k < v.S ? v.top_k : v.S;
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kMaxTopK; ++i)
+            if (i < k) sum += top[i];
+        return sum / (float)k;
+    }
+};
+
+template <int NT, int ST, int STORE, int C>
 __device__ __forceinline__ float cand_cost(const DevView& v, const float* __restrict__ lwin,
                                            int lp, const WinRef& wr, int x, int y, double rx,
                                            double ry, double rz, float d, float nx, float ny,
                                            float nz)
 {
-    constexpr int R = (NT - 1) * ST / 2;
-    constexpr int kMinCount = (NT * NT) / 2;
-    constexpr bool kLocalCoords = NT * NT <= HP3D_LOCAL_TAPS;
-    const double dd = d, dnx = nx, dny = ny, dnz = nz;
-    const double nP = dd * fma(dnx, rx, fma(dny, ry, dnz * rz));
-    if (fabs(nP) < 1e-8) return 2.0f;
-    const double inv = 1.0 / nP;
-    const double* ki = v.kinv_d;
-    // g = K^-T n / (n.P): the reference's factor(p) = g.p
-    const double g0 = fma(ki[0], dnx, fma(ki[3], dny, ki[6] * dnz)) * inv;
-    const double g1 = fma(ki[1], dnx, fma(ki[4], dny, ki[7] * dnz)) * inv;
-    const double g2 = fma(ki[2], dnx, fma(ki[5], dny, ki[8] * dnz)) * inv;
-    const double X = x, Y = y;
-    const double gc = fma(g0, X, fma(g1, Y, g2));   // factor at the window centre
-
-    float top[kMaxTopK];
-#pragma unroll
-    for (int k = 0; k < kMaxTopK; ++k) top[k] = 2.0f;
-
-    const unsigned umax = (unsigned)(v.W - 2), vmax = (unsigned)(v.H - 2);
-    constexpr float kShrink = 0.99999904632568359375f;   // 1 - 2^-20
-    const float Wq = (float)(v.W - 1) * kShrink, Hq = (float)(v.H - 1) * kShrink;
+    CandPlane g;
+    if (!cand_plane(v, x, y, rx, ry, rz, d, nx, ny, nz, g)) return 2.0f;
+    TopCosts t;
     const bool small_k = v.top_k <= 3;   // wave-uniform
-
-    for (int s = 0; s < v.S; ++s) {
-        const double* A = v.src[s].A;
-        const double* b = v.src[s].b;
-        // centre of the window and the two tap-step columns of H
-        const float cx = (float)fma(b[0], gc, fma(A[0], X, fma(A[1], Y, A[2])));
-        const float cy = (float)fma(b[1], gc, fma(A[3], X, fma(A[4], Y, A[5])));
-        const float cz = (float)fma(b[2], gc, fma(A[6], X, fma(A[7], Y, A[8])));
-        const float h00 = (float)fma(b[0], g0, A[0]), h01 = (float)fma(b[0], g1, A[1]);
-        const float h10 = (float)fma(b[1], g0, A[3]), h11 = (float)fma(b[1], g1, A[4]);
-        const float h20 = (float)fma(b[2], g0, A[6]), h21 = (float)fma(b[2], g1, A[7]);
-        const SrcImage<STORE> img(v, s);
-
-        // Small windows' taps relative to an integer base (bu, bv) near the
-        // centre's source position: the base comes out of the centre and the
-        // columns in FP64 (u - bu = (w_x - bu w_z) / w_z, still affine in the
-        // tap offset over w_z), so the taps' FP32 arithmetic works on u - bu,
-        // a few pixels, and rounds to ~ulp(R) instead of ~ulp(u) (1e-5 px at
-        // u ~ 100), an error a 3x3 window's NCC amplifies past 1e-4 of cost.
-        // A centre that projects beyond 2^22 pixels keeps the base 0.
-        float tx = cx, ty = cy, t00 = h00, t01 = h01, t10 = h10, t11 = h11;
-        int bu = 0, bv = 0;
-        if constexpr (kLocalCoords) {
-            const float rc = __builtin_amdgcn_rcpf(cz);
-            const float pu = cx * rc, pv = cy * rc;
-            bu = fabsf(pu) < 4194304.0f ? (int)rintf(pu) : 0;
-            bv = fabsf(pv) < 4194304.0f ? (int)rintf(pv) : 0;
-            const double nu = -(double)bu, nv = -(double)bv;
-            const double CZ = fma(b[2], gc, fma(A[6], X, fma(A[7], Y, A[8])));
-            const double H20 = fma(b[2], g0, A[6]), H21 = fma(b[2], g1, A[7]);
-            tx = (float)fma(nu, CZ, fma(b[0], gc, fma(A[0], X, fma(A[1], Y, A[2]))));
-            t00 = (float)fma(nu, H20, fma(b[0], g0, A[0]));
-            t01 = (float)fma(nu, H21, fma(b[0], g1, A[1]));
-            ty = (float)fma(nv, CZ, fma(b[1], gc, fma(A[3], X, fma(A[4], Y, A[5]))));
-            t10 = (float)fma(nv, H20, fma(b[1], g0, A[3]));
-            t11 = (float)fma(nv, H21, fma(b[1], g1, A[4]));
-        }
-
-        // The unmasked tap loop when every lane's window is inside the
-        // source image (windows with w_z < 0 throughout take the masked
-        // loop, which gives the same result).
-        const bool inside = window_inside(cx, cy, cz, h00, h01, h10, h11, h20, h21, (float)R,
-                                          Wq, Hq);
-        TapSums m;
-        if (__all(inside)) {
-            tap_window<NT, ST, STORE, false, true, RU>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
-                                                       t11, h20, h21, umax, vmax, wr, m, bu, bv);
-        } else if (STORE == kStoreF16 && __all(z_clear(cz, h20, h21, (float)R))) {
-            // FP16 storage only: a third loop without the per-tap |w_z| test
-            // measured +2 % there and -12 % with FP32 storage at stride 1
-            tap_window<NT, ST, STORE, true, false, RU>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
-                                                       t11, h20, h21, umax, vmax, wr, m, bu, bv);
-        } else {
-            tap_window<NT, ST, STORE, true, true, RU>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
-                                                      t11, h20, h21, umax, vmax, wr, m, bu, bv);
-        }
-        const int cnt = m.cnt;
-        const float sr = m.sr, ss = m.ss, srr = m.srr, sss = m.sss, srs = m.srs;
-        float c = 2.0f;
-        if (cnt >= kMinCount) {
-            const double fc = (double)cnt;
-            const double num = fc * (double)srs - (double)sr * (double)ss;
-            const double dr = fc * (double)srr - (double)sr * (double)sr;
-            const double ds = fc * (double)sss - (double)ss * (double)ss;
-            if (!(dr < (double)v.den_eps) && !(ds < (double)v.den_eps)) {
-                // dr, ds >= den_eps (~0.065): far from the denormal range,
-                // where rsqrtf would first rescale, so the bare v_rsq_f32
-                float ncc = (float)num * __builtin_amdgcn_rsqf((float)dr * (float)ds);
-                ncc = fmaxf(-1.0f, fminf(1.0f, ncc));
-                c = 1.0f - ncc;
-            }
-        }
-        // insert into the ascending list of the smallest costs: 3 entries
-        // suffice when at most 3 are averaged (the reference's top-3), else 8
-        if (small_k) {
-#pragma unroll
-            for (int k = 2; k > 0; --k)
-                top[k] = (c < top[k - 1]) ? top[k - 1] : (c < top[k] ? c : top[k]);
-        } else {
-#pragma unroll
-            for (int k = kMaxTopK - 1; k > 0; --k)
-                top[k] = (c < top[k - 1]) ? top[k - 1] : (c < top[k] ? c : top[k]);
-        }
-        top[0] = c < top[0] ? c : top[0];
-    }
-    const int k = v.top_k < v.S ? v.top_k : v.S;
-    float sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kMaxTopK; ++i)
-        if (i < k) sum += top[i];
-    return sum / (float)k;
+    for (int s = 0; s < v.S; ++s)
+        t.insert(source_cost<NT, ST, STORE, C>(v, s, lwin, lp, wr, x, y, g), small_k);
+    return t.mean(v);
 }
 
 // ---------------------------------------------------------------------------
@@ -633,7 +751,7 @@ __device__ __forceinline__ bool cost_pixel(const DevView& v, const float* tile, 
     const float4 h = StateIO<COH>::ld4(v.hyp[parity], p);
     const WinRef wr = window_ref_sums<NT, ST>(lwin, G::LP);
     StateIO<COH>::st1(v.cost[parity], p,
-                      cand_cost<NT, ST, STORE, 1>(v, lwin, G::LP, wr, x, y, rx, ry, rz, h.x, h.y,
+                      cand_cost<NT, ST, STORE, kCostChunk<NT>>(v, lwin, G::LP, wr, x, y, rx, ry, rz, h.x, h.y,
                                                   h.z, h.w));
     return true;
 }
@@ -715,9 +833,28 @@ __device__ __forceinline__ void cost_tile_sorted(const DevView& v, const float* 
         double rx, ry, rz;
         ray_fp64(v.kinv_d, x_o, y_o, rx, ry, rz);
         IO::st1(v.cost[parity], y_o * v.Wc + i_o,
-                cand_cost<NT, ST, STORE, 1>(v, lwin, G::LP, wr, x_o, y_o, rx, ry, rz, hh.x, hh.y,
+                cand_cost<NT, ST, STORE, kCostChunk<NT>>(v, lwin, G::LP, wr, x_o, y_o, rx, ry, rz, hh.x, hh.y,
                                          hh.z, hh.w));
     }
+}
+
+// A refinement candidate: the current hypothesis moved by the draw's four
+// words within the given ranges, its normal normalised and camera-facing
+// (propagate_and_refine_kernel, :610-640).
+__device__ __forceinline__ float4 refine_cand(const float4& best, const uint4& w,
+                                              float depth_range, float normal_range, float dmin,
+                                              float dmax, float ux, float uy, float uz)
+{
+    const float rand_d = u01(w.x) * 2.0f - 1.0f;
+    float cd = best.x + rand_d * depth_range;
+    cd = fmaxf(dmin, fminf(dmax, cd));
+    float cnx = best.y + (u01(w.y) * 2.0f - 1.0f) * normal_range;
+    float cny = best.z + (u01(w.z) * 2.0f - 1.0f) * normal_range;
+    float cnz = best.w + (u01(w.w) * 2.0f - 1.0f) * normal_range;
+    const float nlen = sqrtf(cnx * cnx + cny * cny + cnz * cnz);
+    if (nlen > 1e-12f) { cnx = cnx / nlen; cny = cny / nlen; cnz = cnz / nlen; }
+    if (cnx * ux + cny * uy + cnz * uz > 0.0f) { cnx = -cnx; cny = -cny; cnz = -cnz; }
+    return make_float4(cd, cnx, cny, cnz);
 }
 
 // One pixel of a red (parity 0) or black (parity 1) half-pass:
@@ -894,7 +1031,7 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
             const float4 h = xw.hyp[it];
             double rx, ry, rz;
             ray_fp64(v.kinv_d, x_o, y_o, rx, ry, rz);
-            xw.cost[g] = cand_cost<NT, ST, STORE>(v, tile + ty_o * G::LP + (x_o - 2 * bx * TX),
+            xw.cost[g] = cand_cost<NT, ST, STORE, kPassChunk<NT>>(v, tile + ty_o * G::LP + (x_o - 2 * bx * TX),
                                                   G::LP, wro, x_o, y_o, rx, ry, rz, h.x, h.y, h.z,
                                                   h.w);
         }
@@ -920,18 +1057,11 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
     for (int step = 0; step < 2; ++step) {
         uint32_t c0 = idx, c1 = (uint32_t)iteration, c2 = (uint32_t)step, c3 = kDomainRefine;
         philox(c0, c1, c2, c3, (uint32_t)pass_seed, (uint32_t)(pass_seed >> 32));
-        const float rand_d = u01(c0) * 2.0f - 1.0f;
-        float cd = best.x + rand_d * depth_range;
-        cd = fmaxf(dmin, fminf(dmax, cd));
-        float cnx = best.y + (u01(c1) * 2.0f - 1.0f) * normal_range;
-        float cny = best.z + (u01(c2) * 2.0f - 1.0f) * normal_range;
-        float cnz = best.w + (u01(c3) * 2.0f - 1.0f) * normal_range;
-        const float nlen = sqrtf(cnx * cnx + cny * cny + cnz * cnz);
-        if (nlen > 1e-12f) { cnx = cnx / nlen; cny = cny / nlen; cnz = cnz / nlen; }
-        if (cnx * ux + cny * uy + cnz * uz > 0.0f) { cnx = -cnx; cny = -cny; cnz = -cnz; }
-        const float c = cand_cost<NT, ST, STORE>(v, lwin, G::LP, wr, x, y, rx, ry, rz, cd, cnx,
-                                                 cny, cnz);
-        if (c < bc) { bc = c; best = make_float4(cd, cnx, cny, cnz); changed = true; }
+        const float4 cand = refine_cand(best, make_uint4(c0, c1, c2, c3), depth_range,
+                                        normal_range, dmin, dmax, ux, uy, uz);
+        const float c = cand_cost<NT, ST, STORE, kPassChunk<NT>>(v, lwin, G::LP, wr, x, y, rx, ry, rz, cand.x,
+                                                 cand.y, cand.z, cand.w);
+        if (c < bc) { bc = c; best = cand; changed = true; }
         depth_range *= 0.5f;
         normal_range *= 0.5f;
     }
