@@ -46,18 +46,20 @@ __global__ __launch_bounds__(TX * TY) void pm_cost_kernel(DevView v, int parity,
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
     __shared__ float tile[G::LH * G::LP];
-    __shared__ WaveXchg xw[TX * TY / 64];
+    __shared__ PassXchg<TX * TY> xc;
     int bx, by;
     if (!xcd_tile(tiles_x, tiles, bx, by)) return;
     stage_ref_tile<R, STORE, TX, TY>(v, tile, bx, by);
     cost_tile_sorted<NT, ST, STORE, TX, TY>(v, tile, bx, by, threadIdx.x % TX, threadIdx.x / TX,
-                                            parity, xw[threadIdx.x >> 6]);
+                                            parity, xc);
 }
 
-// Build-time tuning knob of the per-view kernels: minimum waves per SIMD the
-// register allocation must allow (1: no constraint).
+// Minimum waves per SIMD the half-pass's register allocation must allow.  4:
+// every window's kernel fits 128 registers (7 x 7 taps with FP32 planes, 129
+// unasked, keeps three SGPRs' worth of spills outside its loops), and a pass
+// issues a vector instruction nearly every 4 clocks; 5 would spill in the loops.
 #ifndef HP3D_PLAIN_WPE
-#define HP3D_PLAIN_WPE 1
+#define HP3D_PLAIN_WPE 4
 #endif
 
 template <int NT, int ST, int STORE, int TX, int TY>
@@ -68,12 +70,12 @@ void pm_halfpass_kernel(DevView v, int iteration, int parity, uint64_t pass_seed
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
     __shared__ float tile[G::LH * G::LP];
-    __shared__ WaveXchg xw[TX * TY / 64];
+    __shared__ PassXchg<TX * TY> xc;
     int bx, by;
     if (!xcd_tile(tiles_x, tiles, bx, by)) return;
     stage_ref_tile<R, STORE, TX, TY>(v, tile, bx, by);
     halfpass_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, threadIdx.x % TX, threadIdx.x / TX,
-                                          iteration, parity, pass_seed, xw[threadIdx.x >> 6]);
+                                          iteration, parity, pass_seed, xc);
 }
 
 // Colour planes -> row-major depth (H*W), AoS normal (H*W*3), cost and
@@ -220,33 +222,29 @@ hipError_t launch_img_down(const void* prev, int prev_pitch, int W, int H, int s
 }
 
 // Workgroup tile (compacted columns x rows), from sweeps on 1600x1200 views:
-// 32 x 8 (64 x 8 pixels) for windows of up to 8 taps a side (6 x 6 at
-// stride 2: 32x8, 32x4 and 32x2 within 1 %, 16x16 and 64x4 slower); 32 x 4
-// for the 11 x 11 stride-1 window, whose kernel holds 3 waves per SIMD:
-// half-size workgroups leave a shorter tail per launch, +8.5 % with FP32
-// storage (HP3D_PLAIN_TX / _TY override both at build time).
-template <int NT>
-struct PlainTile {
+// 32 x 8 (64 x 8 pixels; 32x4 and 16x16 within 1 % at 6 x 6 taps, 8x32 and
+// 32x16 3 % to 15 % slower; at 11 x 11 taps 32x4, with its shorter lists, 1 to
+// 2 % slower; HP3D_PLAIN_TX / _TY override both at build time).
 #ifdef HP3D_PLAIN_TX
-    static constexpr int TX = HP3D_PLAIN_TX, TY = HP3D_PLAIN_TY;
+constexpr int kPlainTX = HP3D_PLAIN_TX, kPlainTY = HP3D_PLAIN_TY;
 #else
-    static constexpr int TX = 32, TY = NT >= 9 ? 4 : 8;
+constexpr int kPlainTX = 32, kPlainTY = 8;
 #endif
-};
 
 template <int NT, int ST, int STORE>
 static void launch_pass_t(const DevView& v, int mode, int iteration, int parity,
                           uint64_t pass_seed, hipStream_t st)
 {
-    constexpr int kTX = PlainTile<NT>::TX, kTY = PlainTile<NT>::TY;
+    constexpr int kTX = kPlainTX, kTY = kPlainTY;
     const int tiles_x = (v.Wc + kTX - 1) / kTX;
     const int tiles = tiles_x * ((v.H + kTY - 1) / kTY);
     const dim3 grid(((tiles + 7) / 8) * 8);
     // LDS the kernel does not use, to hold fewer workgroups on a CU: the 121-tap
     // initial cost, whose random hypotheses scatter the gathers, thrashes the L1
-    // with the 5 waves to a SIMD that its registers allow (1600x1200, 4 sources,
-    // FP32: 0.48 ms a colour, 0.44 with 3.5; FP16's halved lines: no difference)
-    constexpr unsigned kIdleLds = NT >= 11 && STORE == kStoreF32 ? 6144 : 0;
+    // with the 5 waves to a SIMD that its registers allow (FP32, 4 waves against
+    // 5: 1280x960 with 8 sources 0.584 against 0.602 ms a colour; with FP16's
+    // halved lines no difference)
+    constexpr unsigned kIdleLds = NT >= 11 && STORE == kStoreF32 ? 12288 : 0;
     if (mode == kPassCost)
         hipLaunchKernelGGL((pm_cost_kernel<NT, ST, STORE, kTX, kTY>), grid, dim3(kTX * kTY),
                            kIdleLds, st, v, parity, tiles_x, tiles);

@@ -756,18 +756,58 @@ __device__ __forceinline__ bool cost_pixel(const DevView& v, const float* tile, 
     return true;
 }
 
-// Per-wave LDS scratch of a half-pass: the wave's list of neighbour
-// candidates that must be evaluated (owner lane | candidate << 6), their
-// hypotheses (indexed the same way: each is loaded once, by its owner, and
-// read from here by the lane that evaluates it and by the owner when it
-// accepts it) and their costs, at most 4 per lane; and the depth-bucket
-// counts of the first iteration's ordering.
-struct WaveXchg {
-    unsigned char item[256];
-    float4 hyp[256];
-    float cost[256];
-    int hist[64];
+// Orders a wave's accesses to LDS that no other wave touches: the hardware
+// keeps their order, the fence keeps the compiler's.
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// LDS scratch of a workgroup of T threads in a pass: the list of the neighbour
+// candidates that must be evaluated (owner thread | candidate << 10, at most 4
+// per thread), their hypotheses (by candidate, then owner: each is loaded
+// once, by its owner, and read from here by the lane that evaluates it and by
+// the owner when it accepts it), their costs by list position, the owners'
+// reference sums, and the counts that place entries in the list.
+template <int T> struct PassXchg {
+    static_assert(T % 64 == 0 && T <= 1024, "whole waves, 10 bits of owner thread");
+    unsigned short item[4 * T];
+    float4 hyp[4 * T];
+    float cost[4 * T];
+    WinRef wref[T];
+    int hist[T];        // 64 depth buckets per wave
+    int wsum[T / 64];   // entries per wave
 };
+
+// Depth buckets of a wave's counting sort: inverse depth (disparity) over the
+// view's range.
+struct DepthBuckets {
+    float ilo, iscale;
+    __device__ __forceinline__ DepthBuckets(float dmin, float dmax)
+        : ilo(1.0f / dmax), iscale(64.0f / (1.0f / dmin - ilo)) {}
+    __device__ __forceinline__ int of(float d) const
+    {
+        const int b = (int)((1.0f / d - ilo) * iscale);
+        return b < 0 ? 0 : (b > 63 ? 63 : b);
+    }
+};
+
+// Counts to places: on return hist[b] is the sum of the wave's counts below b.
+__device__ __forceinline__ void scan_buckets(int* hist, int lane)
+{
+    wave_lds_order();
+    const int cnt = hist[lane];
+    int incl = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int u = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += u;
+    }
+    wave_lds_order();
+    hist[lane] = incl - cnt;
+    wave_lds_order();
+}
 
 // Cost of the current hypotheses of colour `parity` at this workgroup's
 // pixels (compute_ncc_cost_kernel, patchmatch_mvs.cu:349-513), evaluated in
@@ -775,56 +815,44 @@ struct WaveXchg {
 // lane's windows would gather from an unrelated part of every source; a
 // counting sort of the wave's hypotheses by inverse depth (disparity) hands
 // lane k the k-th, so a wave's gathers fall in a narrower band of each
-// source.  Any lane can evaluate any pixel's candidate (the whole window
+// source.  (Sorted over the whole workgroup the bands are narrower still, but
+// a wave's pixels spread over the tile: 0.149 -> 0.155 ms a colour at
+// 1600x1200.)  Any lane can evaluate any pixel's candidate (the whole window
 // tile is in LDS) and a cost is a pure function of the pixel and the
-// hypothesis, so the result is the same as one lane per pixel.  Every
-// thread of the workgroup must call this (it synchronises the group).
+// hypothesis, so the result is the same as one lane per pixel.
 template <int NT, int ST, int STORE, int TX, int TY, bool COH = false>
 __device__ __forceinline__ void cost_tile_sorted(const DevView& v, const float* tile, int bx,
-                                                 int by, int tx, int ty, int parity, WaveXchg& xw)
+                                                 int by, int tx, int ty, int parity,
+                                                 PassXchg<TX * TY>& xc)
 {
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
     using IO = StateIO<COH>;
-    constexpr int kBuckets = 64;
-    const int lane = threadIdx.x & 63;
-    const int wave0 = threadIdx.x & ~63;
+    const int t = threadIdx.x, lane = t & 63, wave0 = t & ~63;
     const int i = bx * TX + tx, y = by * TY + ty;
     const int x = 2 * i + ((y + parity) & 1);
     const bool active = y < v.H && x < v.W;
     float4 h = make_float4(0.f, 0.f, 0.f, 0.f);
     if (active) h = IO::ld4(v.hyp[parity], y * v.Wc + i);
-    xw.hist[lane] = 0;
-    __builtin_amdgcn_wave_barrier();
+    int* hist = xc.hist + wave0;
+    hist[lane] = 0;
+    wave_lds_order();
     int bk = 0, rk = 0;
     if (active) {
-        const float ilo = 1.0f / v.dmax, iscale = (float)kBuckets / (1.0f / v.dmin - ilo);
-        const int b = (int)((1.0f / h.x - ilo) * iscale);
-        bk = b < 0 ? 0 : (b > kBuckets - 1 ? kBuckets - 1 : b);
-        rk = atomicAdd(&xw.hist[bk], 1);
+        bk = DepthBuckets(v.dmin, v.dmax).of(h.x);
+        rk = atomicAdd(&hist[bk], 1);
     }
-    __builtin_amdgcn_wave_barrier();
-    const int cnt = xw.hist[lane];
-    int incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int t = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += t;
-    }
-    __builtin_amdgcn_wave_barrier();
-    xw.hist[lane] = incl - cnt;
-    __builtin_amdgcn_wave_barrier();
+    scan_buckets(hist, lane);
     if (active) {
-        const int slot = xw.hist[bk] + rk;
-        xw.item[slot] = (unsigned char)lane;
-        xw.hyp[slot] = h;
+        const int slot = wave0 + hist[bk] + rk;
+        xc.item[slot] = (unsigned short)t;
+        xc.hyp[slot] = h;
     }
-    const unsigned total = (unsigned)__popcll(__ballot(active));
-    __syncthreads();
-    if ((unsigned)lane < total) {
-        const int ol = xw.item[lane];
-        const float4 hh = xw.hyp[lane];
-        const int t_o = wave0 + ol;
+    const int total = __popcll(__ballot(active));
+    wave_lds_order();
+    if (lane < total) {
+        const int t_o = xc.item[t];
+        const float4 hh = xc.hyp[t];
         const int tx_o = t_o % TX, ty_o = t_o / TX;
         const int i_o = bx * TX + tx_o, y_o = by * TY + ty_o;
         const int x_o = 2 * i_o + ((y_o + parity) & 1);
@@ -833,8 +861,8 @@ __device__ __forceinline__ void cost_tile_sorted(const DevView& v, const float* 
         double rx, ry, rz;
         ray_fp64(v.kinv_d, x_o, y_o, rx, ry, rz);
         IO::st1(v.cost[parity], y_o * v.Wc + i_o,
-                cand_cost<NT, ST, STORE, kCostChunk<NT>>(v, lwin, G::LP, wr, x_o, y_o, rx, ry, rz, hh.x, hh.y,
-                                         hh.z, hh.w));
+                cand_cost<NT, ST, STORE, kCostChunk<NT>>(v, lwin, G::LP, wr, x_o, y_o, rx, ry, rz,
+                                                         hh.x, hh.y, hh.z, hh.w));
     }
 }
 
@@ -868,23 +896,22 @@ __device__ __forceinline__ float4 refine_cand(const float4& best, const uint4& w
 // deterministic function of (pixel, hypothesis), and bc is already at most
 // that cost.  Once propagation has spread planes, 40-60 % of the neighbour
 // candidates are such repeats, but rarely all 64 lanes of a wave at once.  So
-// the wave lists the candidates its lanes still need (also leaving out
+// the workgroup lists the candidates its lanes still need (also leaving out
 // neighbours unchanged since this pixel's previous pass, see below), any
 // lane evaluates any
 // pixel's candidate (all windows of the workgroup are in LDS), and each
 // owner then applies the costs in L, R, U, D order.  The result is the one
-// the plain per-lane loop gives, with fewer evaluation rounds per wave.
+// the plain per-lane loop gives, with fewer evaluation rounds.
 // Every thread of the workgroup must call this (it synchronises the group).
 template <int NT, int ST, int STORE, int TX, int TY, bool COH = false>
 __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* tile, int bx, int by,
                                                int tx, int ty, int iteration, int parity,
-                                               uint64_t pass_seed, WaveXchg& xw)
+                                               uint64_t pass_seed, PassXchg<TX * TY>& xc)
 {
-    constexpr int R = (NT - 1) * ST / 2;
+    constexpr int R = (NT - 1) * ST / 2, T = TX * TY;
     using G = TileGeom<R, STORE, TX, TY>;
     using IO = StateIO<COH>;
-    const int lane = threadIdx.x & 63;
-    const int wave0 = threadIdx.x & ~63;
+    const int t = threadIdx.x, lane = t & 63, wave0 = t & ~63;
     const int i = bx * TX + tx;
     const int y = by * TY + ty;
     const int o = (y + parity) & 1;
@@ -942,98 +969,95 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
             for (int j = 0; j < k; ++j) n = n && !(ok[j] && same(h[j], h[k]));
             need |= (unsigned)n << k;
             hd[k] = h[k].x;
-            if (n) xw.hyp[lane | (k << 6)] = h[k];
+            if (n) xc.hyp[t + k * T] = h[k];
         }
     }
     const WinRef wr = window_ref_sums<NT, ST>(lwin, G::LP);
+    xc.wref[t] = wr;
 
-    // Wave-wide list ordered by owner lane, then candidate: a round of 64
-    // items then covers ~25 neighbouring pixels whose candidates project to
+    // The workgroup's list, ordered by owner thread, then candidate: a round of
+    // 64 items then covers neighbouring pixels whose candidates project to
     // nearly the same source rows and columns, so its gathers touch far
-    // fewer 64-B segments than 64 pixels' worth would (the L1 access rate,
-    // not bandwidth, bounds this kernel).
+    // fewer 64-B segments than 64 pixels' worth would.  The waves take its
+    // rounds in turn: per wave, the last round would on average be half empty,
+    // half of the 3 to 4 rounds a converged pass has (1600x1200, 4 sources,
+    // stride 2: 0.446 -> 0.427 ms a half-pass; 1280x960, 8 sources, stride 1:
+    // 1.77 -> 1.68 ms; with 512 threads 3 % slower again).
     const unsigned long long below = (1ull << lane) - 1ull;
     int slot[4];
-    unsigned total = 0;
-    int base = 0;   // items of the lanes below this one
+    int base = 0, count = 0;   // entries of the lanes below this one, of the wave
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const unsigned long long m = __ballot((need >> k) & 1u);
         base += __popcll(m & below);
-        total += (unsigned)__popcll(m);
+        count += __popcll(m);
     }
+    if (lane == 0) xc.wsum[t >> 6] = count;
+    bool sorted = false;
 #if HP3D_BUCKET
     if (NT < 9 && iteration < v.first_iteration + HP3D_BUCKET) {
         // First iteration: the neighbours hold random, unrelated depths, so
-        // owner order does not cluster the gathers.  Order the items by
-        // inverse depth (disparity) instead, in kBuckets buckets (a counting
-        // sort in LDS; the order within a bucket does not matter), so each
-        // round's windows lie in a narrower band of every source.  (+1.4 %
-        // on 6x6-tap windows; with 11x11 windows it measured slower.)
-        constexpr int kBuckets = 64;
-        const float ilo = 1.0f / dmax, iscale = (float)kBuckets / (1.0f / dmin - ilo);
-        xw.hist[lane] = 0;
-        __builtin_amdgcn_wave_barrier();
+        // owner order does not cluster the gathers.  Order each wave's entries
+        // by inverse depth (disparity) instead (the order within a bucket does
+        // not matter), so a round's windows lie in a narrower band of every
+        // source.  (+1.4 % on 6x6-tap windows; with 11x11 windows it measured
+        // slower, and so did sorting over the workgroup: 0.744 -> 0.818 ms.)
+        int* hist = xc.hist + wave0;
+        const DepthBuckets db(dmin, dmax);
+        hist[lane] = 0;
+        wave_lds_order();
         int bk[4], rk[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             bk[k] = 0;
             rk[k] = 0;
             if ((need >> k) & 1u) {
-                const int b = (int)((1.0f / hd[k] - ilo) * iscale);
-                bk[k] = b < 0 ? 0 : (b > kBuckets - 1 ? kBuckets - 1 : b);
-                rk[k] = atomicAdd(&xw.hist[bk[k]], 1);
+                bk[k] = db.of(hd[k]);
+                rk[k] = atomicAdd(&hist[bk[k]], 1);
             }
         }
-        __builtin_amdgcn_wave_barrier();
-        const int cnt = xw.hist[lane];
-        int incl = cnt;
+        scan_buckets(hist, lane);
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int t = __shfl_up(incl, d, 64);
-            if (lane >= d) incl += t;
-        }
-        __builtin_amdgcn_wave_barrier();
-        xw.hist[lane] = incl - cnt;
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            slot[k] = 0;
-            if ((need >> k) & 1u) {
-                slot[k] = xw.hist[bk[k]] + rk[k];
-                xw.item[slot[k]] = (unsigned char)(lane | (k << 6));
-            }
-        }
-    } else
+        for (int k = 0; k < 4; ++k) slot[k] = hist[bk[k]] + rk[k];
+        sorted = true;
+    }
 #endif
-    {
-        int off = base;
+    if (!sorted) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            slot[k] = off;
-            if ((need >> k) & 1u) {
-                xw.item[off] = (unsigned char)(lane | (k << 6));
-                ++off;
-            }
+            slot[k] = base;
+            base += (need >> k) & 1u;
         }
     }
     __syncthreads();
-    for (unsigned r = 0; r < total; r += 64) {
-        const unsigned g = r + lane;
-        const unsigned it = xw.item[g < total ? g : total - 1];
-        const int ol = it & 63;
-        const WinRef wro{__shfl(wr.sr, ol, 64), __shfl(wr.srr, ol, 64)};
+    int first = 0, total = 0;   // this wave's first entry, the workgroup's entries
+#pragma unroll
+    for (int w = 0; w < T / 64; ++w) {
+        const int c = xc.wsum[w];
+        if (w < (t >> 6)) first += c;
+        total += c;
+    }
+    total = __builtin_amdgcn_readfirstlane(total);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        slot[k] += first;
+        if ((need >> k) & 1u) xc.item[slot[k]] = (unsigned short)(t | (k << 10));
+    }
+    __syncthreads();
+    for (int g0 = __builtin_amdgcn_readfirstlane(wave0); g0 < total; g0 += T) {
+        const int g = g0 + lane;
         if (g < total) {
-            const int t_o = wave0 + ol;
+            const unsigned it = xc.item[g];
+            const int t_o = it & 1023;
             const int tx_o = t_o % TX, ty_o = t_o / TX;
             const int i_o = bx * TX + tx_o, y_o = by * TY + ty_o;
             const int o_o = (y_o + parity) & 1, x_o = 2 * i_o + o_o;
-            const float4 h = xw.hyp[it];
+            const float4 h = xc.hyp[t_o + (int)(it >> 10) * T];
             double rx, ry, rz;
             ray_fp64(v.kinv_d, x_o, y_o, rx, ry, rz);
-            xw.cost[g] = cand_cost<NT, ST, STORE, kPassChunk<NT>>(v, tile + ty_o * G::LP + (x_o - 2 * bx * TX),
-                                                  G::LP, wro, x_o, y_o, rx, ry, rz, h.x, h.y, h.z,
-                                                  h.w);
+            xc.cost[g] = cand_cost<NT, ST, STORE, kPassChunk<NT>>(
+                v, tile + ty_o * G::LP + (x_o - 2 * bx * TX), G::LP, xc.wref[t_o], x_o, y_o, rx,
+                ry, rz, h.x, h.y, h.z, h.w);
         }
     }
     __syncthreads();
@@ -1041,8 +1065,8 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (!((need >> k) & 1u)) continue;
-        const float c = xw.cost[slot[k]];
-        if (c < bc) { bc = c; best = xw.hyp[lane | (k << 6)]; changed = true; }
+        const float c = xc.cost[slot[k]];
+        if (c < bc) { bc = c; best = xc.hyp[t + k * T]; changed = true; }
     }
 
     double rx, ry, rz;

@@ -30,16 +30,19 @@ namespace hp3d {
 
 constexpr int kStepChunk = 16;   // tiles per chunk of the XCD interleave
 constexpr int kPersistMaxGrid = 4096;
+// Waves per SIMD that every step kernel's registers must allow (128): only the
+// 11-tap FP32 instances need asking (134 registers without), and do not spill.
+constexpr int kStepWaves = 4;
 
 template <int NT, int ST, int STORE, int TX, int TY, int WPE>
-__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE < kStepWaves ? kStepWaves : WPE, 8)))
 void pm_step_kernel(const DevJob* __restrict__ jobs, const StepItem* __restrict__ items,
                     int n_items, int total_tiles)
 {
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
     __shared__ float tile[G::LH * G::LP];
-    __shared__ WaveXchg xw[TX * TY / 64];
+    __shared__ PassXchg<TX * TY> xc;
 
     const int b = blockIdx.x;                       // gridDim.x: a multiple of 8 * kStepChunk
     const int sidx = b >> 3;                        // position in this XCD's sequence
@@ -71,7 +74,7 @@ void pm_step_kernel(const DevJob* __restrict__ jobs, const StepItem* __restrict_
         cost_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, tx, ty, 1);
     } else {
         halfpass_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, tx, ty, it.iteration, it.parity,
-                                              it.pass_seed, xw[threadIdx.x >> 6]);
+                                              it.pass_seed, xc);
     }
     // outputs: this lane's pixel of each colour; the other colour was
     // completed by the previous step
@@ -133,7 +136,7 @@ void pm_persist_kernel(const DevJob* __restrict__ jobs, const StepItem* __restri
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
     __shared__ float tile[G::LH * G::LP];
-    __shared__ WaveXchg xw[TX * TY / 64];
+    __shared__ PassXchg<TX * TY> xc;
     __shared__ int s_word;
     int* const ctl = done + n_counters;
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
@@ -233,7 +236,7 @@ void pm_persist_kernel(const DevJob* __restrict__ jobs, const StepItem* __restri
             } else {
                 halfpass_pixel<NT, ST, STORE, TX, TY, true>(v, tile, bx, by, tx, ty, it.iteration,
                                                             it.parity, it.pass_seed,
-                                                            xw[threadIdx.x >> 6]);
+                                                            xc);
             }
             if (it.emit && y < v.H) {
                 for (int c = 0; c < 2; ++c) {
