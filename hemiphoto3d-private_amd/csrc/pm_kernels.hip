@@ -22,6 +22,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "pm_device.h"
 #include "pm_launch.h"
 #include "pm_pixel.h"
@@ -37,21 +39,21 @@ __global__ __launch_bounds__(256) void pm_init_kernel(DevView v, uint64_t seed)
     v.hyp[(x + y) & 1][y * v.Wc + (x >> 1)] = init_hyp(v, x, y, seed);
 }
 
-// Cost of the current hypotheses of one colour, run once per colour before
-// the first iteration.
+// Cost of the current hypotheses, run once before the first iteration: the two
+// colours of a tile by neighbouring workgroups.
 template <int NT, int ST, int STORE, int TX, int TY>
-__global__ __launch_bounds__(TX * TY) void pm_cost_kernel(DevView v, int parity, int tiles_x,
-                                                          int tiles)
+__global__ __launch_bounds__(TX * TY) void pm_cost_kernel(DevView v, int tiles_x, int tiles)
 {
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
     __shared__ float tile[G::LH * G::LP];
     __shared__ PassXchg<TX * TY> xc;
-    int bx, by;
-    if (!xcd_tile(tiles_x, tiles, bx, by)) return;
+    int t;
+    if (!xcd_unit(2 * tiles, t)) return;
+    const int by = (t >> 1) / tiles_x, bx = (t >> 1) - by * tiles_x;
     stage_ref_tile<R, STORE, TX, TY>(v, tile, bx, by);
     cost_tile_sorted<NT, ST, STORE, TX, TY>(v, tile, bx, by, threadIdx.x % TX, threadIdx.x / TX,
-                                            parity, xc);
+                                            t & 1, xc);
 }
 
 // Minimum waves per SIMD the half-pass's register allocation must allow.  4:
@@ -76,6 +78,33 @@ void pm_halfpass_kernel(DevView v, int iteration, int parity, uint64_t pass_seed
     stage_ref_tile<R, STORE, TX, TY>(v, tile, bx, by);
     halfpass_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, threadIdx.x % TX, threadIdx.x / TX,
                                           iteration, parity, pass_seed, xc);
+}
+
+// Views of few pixels: up to kMaxSplitWaves waves for 64 pixels (halfpass_split).
+template <int NT, int ST, int STORE, int TX, int TY>
+__global__ __launch_bounds__(64 * kMaxSplitWaves)
+void pm_halfpass_split_kernel(DevView v, int iteration, int parity, uint64_t pass_seed,
+                              int tiles_x, int tiles)
+{
+    using G = TileGeom<(NT - 1) * ST / 2, STORE, TX, TY>;
+    __shared__ float tile[G::LH * G::LP];
+    __shared__ SplitXchg xs;
+    int bx, by;
+    if (!xcd_tile(tiles_x, tiles, bx, by)) return;
+    halfpass_split<NT, ST, STORE, TX, TY>(v, tile, bx, by, iteration, parity, pass_seed, xs);
+}
+
+template <int NT, int ST, int STORE, int TX, int TY>
+__global__ __launch_bounds__(64 * kMaxSrc)
+void pm_cost_split_kernel(DevView v, int tiles_x, int tiles)
+{
+    using G = TileGeom<(NT - 1) * ST / 2, STORE, TX, TY>;
+    __shared__ float tile[G::LH * G::LP];
+    __shared__ SplitXchg xs;
+    int t;
+    if (!xcd_unit(2 * tiles, t)) return;
+    const int by = (t >> 1) / tiles_x, bx = (t >> 1) - by * tiles_x;
+    cost_split<NT, ST, STORE, TX, TY>(v, tile, bx, by, t & 1, xs);
 }
 
 // Colour planes -> row-major depth (H*W), AoS normal (H*W*3), cost and
@@ -231,14 +260,59 @@ constexpr int kPlainTX = HP3D_PLAIN_TX, kPlainTY = HP3D_PLAIN_TY;
 constexpr int kPlainTX = 32, kPlainTY = 8;
 #endif
 
+// The split kernels' tile: 16 x 4 (32 x 4 pixels; 32x2 and 8x8 within 3 %).
+constexpr int kSplitTX = 16, kSplitTY = 4;
+
+// Waves of a split workgroup for a view of n such tiles, 0: not split.  Split,
+// every wave repeats the pixel's bookkeeping and the rounds are not pooled, so
+// it pays only while the plain kernel's n / 4 workgroups leave SIMDs idle for
+// the length of their chain of S sources: up to n = 400 S for windows of up to
+// 49 taps, 750 S above.  Half-pass, plain -> split, at and beyond the line:
+//   6x6 taps: 480x360 S=8 0.161 -> 0.123 ms, 560x420 S=4 0.092 -> 0.093,
+//             641x479 S=5 0.139 -> 0.143, 800x600 S=8 0.268 -> 0.283
+//   11x11:    480x360 S=2 0.135 -> 0.120, 560x420 S=2 0.140 -> 0.151,
+//             800x600 S=6 0.617 -> 0.604, 1280x960 S=5 1.217 -> 1.254
+// 4 waves a workgroup fill a CU best (S = 5 with 6: a CU holds 2 such
+// workgroups, 12 of its 16 waves; +20 %); the smallest views, whose waves do
+// not fill the chip at 8 a workgroup either, are fastest with 8, and with room
+// for both refinement steps (3 S) below 160 tiles.  96x72, S=8, 6x6 taps:
+// 0.138 ms plain, 0.054 with 4 waves, 0.039 with 8, 0.036 with 16.
+static int split_waves(int NT, int n, int S)
+{
+    if (n > (NT * NT >= 81 ? 750 : 400) * S) return 0;
+    return n > 300 ? 4 : n > 160 ? 8 : std::min(kMaxSplitWaves, std::max(8, 3 * S));
+}
+
+// The same for the initial cost, whose workgroups have no chain but the
+// sources: up to n = 1600 S (800x600, S=6, 11x11: 0.400 -> 0.322 ms for both
+// colours, 1280x960 S=8 1.18 -> 1.05, S=3 at 6x6 0.153 -> 0.154, 1600x1200 S=4
+// 0.286 -> 0.320).
+static int cost_split_waves(int n, int S)
+{
+    if (n > 1600 * S || S < 2) return 0;
+    return std::min(n > 300 ? 4 : 8, S);
+}
+
 template <int NT, int ST, int STORE>
 static void launch_pass_t(const DevView& v, int mode, int iteration, int parity,
                           uint64_t pass_seed, hipStream_t st)
 {
+    const int sx = (v.Wc + kSplitTX - 1) / kSplitTX, sn = sx * ((v.H + kSplitTY - 1) / kSplitTY);
+    const int waves = mode == kPassCost ? cost_split_waves(sn, v.S) : split_waves(NT, sn, v.S);
+    if (waves && mode == kPassCost) {
+        hipLaunchKernelGGL((pm_cost_split_kernel<NT, ST, STORE, kSplitTX, kSplitTY>),
+                           dim3(xcd_grid(2 * sn)), dim3(64 * waves), 0, st, v, sx, sn);
+        return;
+    }
+    if (waves) {
+        hipLaunchKernelGGL((pm_halfpass_split_kernel<NT, ST, STORE, kSplitTX, kSplitTY>),
+                           dim3(xcd_grid(sn)), dim3(64 * waves), 0, st, v, iteration, parity,
+                           pass_seed, sx, sn);
+        return;
+    }
     constexpr int kTX = kPlainTX, kTY = kPlainTY;
     const int tiles_x = (v.Wc + kTX - 1) / kTX;
     const int tiles = tiles_x * ((v.H + kTY - 1) / kTY);
-    const dim3 grid(((tiles + 7) / 8) * 8);
     // LDS the kernel does not use, to hold fewer workgroups on a CU: the 121-tap
     // initial cost, whose random hypotheses scatter the gathers, thrashes the L1
     // with the 5 waves to a SIMD that its registers allow (FP32, 4 waves against
@@ -246,11 +320,11 @@ static void launch_pass_t(const DevView& v, int mode, int iteration, int parity,
     // halved lines no difference)
     constexpr unsigned kIdleLds = NT >= 11 && STORE == kStoreF32 ? 12288 : 0;
     if (mode == kPassCost)
-        hipLaunchKernelGGL((pm_cost_kernel<NT, ST, STORE, kTX, kTY>), grid, dim3(kTX * kTY),
-                           kIdleLds, st, v, parity, tiles_x, tiles);
+        hipLaunchKernelGGL((pm_cost_kernel<NT, ST, STORE, kTX, kTY>), dim3(xcd_grid(2 * tiles)),
+                           dim3(kTX * kTY), kIdleLds, st, v, tiles_x, tiles);
     else
-        hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY>), grid, dim3(kTX * kTY), 0,
-                           st, v, iteration, parity, pass_seed, tiles_x, tiles);
+        hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY>), dim3(xcd_grid(tiles)),
+                           dim3(kTX * kTY), 0, st, v, iteration, parity, pass_seed, tiles_x, tiles);
 }
 
 template <int STORE>

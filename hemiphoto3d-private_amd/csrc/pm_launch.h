@@ -27,7 +27,8 @@ hipError_t launch_img_down(const void* prev, int prev_pitch, int W, int H, int s
 // W*H ints of scratch.
 hipError_t launch_seed(const DevView& v, const hp3d_seed_point* seeds, int n, int radius,
                        int* owner, hipStream_t st);
-// mode kPassCost: cost of the current hypotheses of colour `parity`;
+// mode kPassCost: cost of the current hypotheses of both colours (iteration,
+// parity and pass_seed unused);
 // mode kPassPropagate: one half-pass of colour `parity` at `iteration`.
 hipError_t launch_pass(const DevView& v, int store, int radius, int stride, int mode,
                        int iteration, int parity, uint64_t pass_seed, hipStream_t st);

@@ -116,8 +116,8 @@ extern "C" int hp3d_pm_run_view_noalloc(hp3d_pm_ctx* ctx, const hp3d_view_desc* 
 
     // the launch sequence of hp3d_pm_run_view, without timing events
     hipError_t e = launch_init(v, d->seed, ctx->stream);
-    for (int parity = 0; parity < 2 && e == hipSuccess; ++parity)
-        e = launch_pass(v, ref->store, d->radius, d->stride, kPassCost, 0, parity, 0, ctx->stream);
+    if (e == hipSuccess)
+        e = launch_pass(v, ref->store, d->radius, d->stride, kPassCost, 0, 0, 0, ctx->stream);
     for (int it = d->first_iteration; it < d->first_iteration + d->iterations && e == hipSuccess;
          ++it)
         for (int parity = 0; parity < 2 && e == hipSuccess; ++parity)

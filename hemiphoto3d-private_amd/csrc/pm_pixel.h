@@ -698,12 +698,13 @@ struct TileGeom {
 // Tile (bx, by) covers compacted columns bx*TX .. bx*TX+TX-1 (pixel columns
 // 2*bx*TX .. 2*bx*TX+2*TX-1) of rows by*TY .. by*TY+TY-1.
 template <int R, int STORE, int TX, int TY>
-__device__ __forceinline__ void stage_ref_tile(const DevView& v, float* tile, int bx, int by)
+__device__ __forceinline__ void stage_ref_tile(const DevView& v, float* tile, int bx, int by,
+                                               int threads = TX * TY)
 {
     using G = TileGeom<R, STORE, TX, TY>;
     const int X0 = 2 * bx * TX - R;
     const int Y0 = by * TY - R;
-    for (int k = threadIdx.x; k < G::LW * G::LH; k += TX * TY) {
+    for (int k = threadIdx.x; k < G::LW * G::LH; k += threads) {
         const int ly = k / G::LW, lx = k - ly * G::LW;
         const int gx = min(max(X0 + lx, 0), v.W - 1);
         const int gy = min(max(Y0 + ly, 0), v.H - 1);
@@ -1092,6 +1093,241 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
     IO::st4(own, p, best);
     IO::st1(v.cost[parity], p, bc);
     IO::stb(v.chg[parity], p, changed ? 1u : 0u);
+}
+
+// ---------------------------------------------------------------------------
+// The same passes for views of few pixels: a workgroup of up to kMaxSplitWaves
+// waves takes the 64 pixels of one colour in a tile (TX * TY = 64), and its
+// waves share the evaluations, one (64 candidates, source) at a time.  A
+// source's cost is a pure function of (pixel, hypothesis, source) and goes to
+// its place in LDS, so the costs, and the means over the smallest of them, are
+// the bits one lane per pixel gives.
+//
+// What bounds such a view is the chain of evaluations that one wave of
+// halfpass_pixel does one after another, up to 6 candidates x S sources, while
+// most of the 1024 SIMDs have no wave (a 96x72 view has 54).  With a wave per
+// source the chain is 4 + 1 + 1 evaluations; with 4 S waves the rounds of
+// neighbours run side by side too, and with 3 S the two refinement steps: the
+// second is evaluated for both outcomes of the first.
+// ---------------------------------------------------------------------------
+constexpr int kMaxSplitWaves = 16;
+
+struct SplitXchg {
+    unsigned char item[256];               // listed neighbours: owner lane | candidate << 6
+    float4 hyp[256];                       // their hypotheses, by the same index
+    float cost[kMaxSrc][256];              // source costs by list position
+    float cost_r[3][kMaxSrc][64];          // source costs of the refinement candidates
+    uint4 rnd[2][64];                      // the refinement steps' Philox words
+};
+
+// Mean of the smallest source costs at position g.
+template <int N>
+__device__ __forceinline__ float split_mean(const DevView& v, const float (*cost)[N], int g)
+{
+    TopCosts t;
+    const bool small_k = v.top_k <= 3;
+    for (int s = 0; s < v.S; ++s) t.insert(cost[s][g], small_k);
+    return t.mean(v);
+}
+
+template <int NT, int ST, int STORE, int TX, int TY>
+__device__ __forceinline__ void halfpass_split(const DevView& v, float* tile, int bx, int by,
+                                               int iteration, int parity, uint64_t pass_seed,
+                                               SplitXchg& xs)
+{
+    static_assert(TX * TY == 64, "one wave of pixels per tile");
+    constexpr int R = (NT - 1) * ST / 2;
+    using G = TileGeom<R, STORE, TX, TY>;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int waves = (int)blockDim.x >> 6;
+    const int tx = lane % TX, ty = lane / TX;
+    const int i = bx * TX + tx, y = by * TY + ty;
+    const int o = (y + parity) & 1, x = 2 * i + o;
+    const bool active = y < v.H && x < v.W;
+    const float dmin = v.dmin, dmax = v.dmax;
+    const int Wc = v.Wc, p = y * Wc + i;
+    auto same = [](const float4& a, const float4& b) {
+        return __float_as_uint(a.x) == __float_as_uint(b.x) &&
+               __float_as_uint(a.y) == __float_as_uint(b.y) &&
+               __float_as_uint(a.z) == __float_as_uint(b.z) &&
+               __float_as_uint(a.w) == __float_as_uint(b.w);
+    };
+    stage_ref_tile<R, STORE, TX, TY>(v, tile, bx, by, (int)blockDim.x);
+    if (wave == waves - 1) {
+        // the refinement draws depend on no hypothesis
+#pragma unroll 1
+        for (int step = 0; step < 2; ++step) {
+            uint32_t c0 = (uint32_t)(y * v.W + x), c1 = (uint32_t)iteration, c2 = (uint32_t)step;
+            uint32_t c3 = kDomainRefine;
+            philox(c0, c1, c2, c3, (uint32_t)pass_seed, (uint32_t)(pass_seed >> 32));
+            xs.rnd[step][lane] = make_uint4(c0, c1, c2, c3);
+        }
+    }
+    // every wave holds its lane's pixel: which neighbours have to be evaluated
+    // (the conditions of halfpass_pixel) and where they are listed
+    float4 best = make_float4(0.f, 0.f, 0.f, 0.f);
+    float bc = 2.0f;
+    unsigned need = 0;
+    if (active) {
+        const float4* oth = v.hyp[parity ^ 1];
+        const unsigned char* chg_oth = v.chg[parity ^ 1];
+        best = v.hyp[parity][p];
+        bc = v.cost[parity][p];
+        const bool seen = iteration > v.first_iteration;
+        float4 h[4];
+        bool ok[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bool has = k == 0 ? x >= 1 : k == 1 ? x + 1 < v.W : k == 2 ? y >= 1 : y + 1 < v.H;
+            const int q = k == 0 ? p + o - 1 : k == 1 ? p + o : k == 2 ? p - Wc : p + Wc;
+            ok[k] = false;
+            h[k] = best;
+            bool stale = false;
+            if (has) {
+                h[k] = oth[q];
+                ok[k] = !(h[k].x < dmin || h[k].x > dmax);
+                stale = seen && chg_oth[q] == 0;
+            }
+            bool n = ok[k] && !stale && !same(h[k], best);
+#pragma unroll
+            for (int j = 0; j < k; ++j) n = n && !(ok[j] && same(h[j], h[k]));
+            need |= (unsigned)n << k;
+            if (n && wave == 0) xs.hyp[lane | (k << 6)] = h[k];
+        }
+    }
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int base = 0, total = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const unsigned long long m = __ballot((need >> k) & 1u);
+        base += __popcll(m & below);
+        total += __popcll(m);
+    }
+    if (wave == 0) {
+        int off = base;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if ((need >> k) & 1u) xs.item[off++] = (unsigned char)(lane | (k << 6));
+    }
+    __syncthreads();
+    const float* lwin = tile + ty * G::LP + (x - 2 * bx * TX);
+    const WinRef wr = window_ref_sums<NT, ST>(lwin, G::LP);
+    float ux, uy, uz;
+    unit_ray(v.kinv, x, y, ux, uy, uz);
+    float depth_range = (dmax - dmin) * 0.5f, normal_range = 1.0f;
+    for (int it = 0; it < iteration; ++it) { depth_range *= 0.6f; normal_range *= 0.6f; }
+    // the refinement candidate of a step from hypothesis h
+    auto draw = [&](int step, const float4& h) {
+        const float f = step ? 0.5f : 1.0f;
+        return refine_cand(h, xs.rnd[step][lane], depth_range * f, normal_range * f, dmin, dmax,
+                           ux, uy, uz);
+    };
+    // phase 0: the listed neighbours, 64 a round; phase 1: the first refinement
+    // step and, with the waves for it, the second step from either outcome;
+    // phase 2: else the second step
+    const bool both = waves >= 3 * v.S;
+    bool changed = false;
+#pragma unroll 1
+    for (int phase = 0; phase < 3; ++phase) {
+        const int groups = phase == 0 ? (total + 63) >> 6 : phase == 1 && both ? 3 : 1;
+#pragma unroll 1
+        for (int u = wave; u < groups * v.S; u += waves) {
+            const int r = u / v.S, s = u - r * v.S;
+            int ol = lane;
+            bool on = active;
+            float4 h;
+            if (phase == 0) {
+                on = r * 64 + lane < total;
+                const unsigned it = xs.item[on ? r * 64 + lane : total - 1];
+                ol = it & 63;
+                h = xs.hyp[it];
+            } else {
+                h = draw(phase == 2 || r == 1 ? 1 : 0, best);
+                if (r == 2) h = draw(1, h);
+            }
+            const WinRef wro{__shfl(wr.sr, ol, 64), __shfl(wr.srr, ol, 64)};
+            if (on) {
+                const int tx_o = ol % TX, ty_o = ol / TX;
+                const int i_o = bx * TX + tx_o, y_o = by * TY + ty_o;
+                const int x_o = 2 * i_o + ((y_o + parity) & 1);
+                double rx, ry, rz;
+                ray_fp64(v.kinv_d, x_o, y_o, rx, ry, rz);
+                CandPlane cp;
+                float c = 2.0f;
+                if (cand_plane(v, x_o, y_o, rx, ry, rz, h.x, h.y, h.z, h.w, cp))
+                    c = source_cost<NT, ST, STORE, kPassChunk<NT>>(
+                        v, s, tile + ty_o * G::LP + (x_o - 2 * bx * TX), G::LP, wro, x_o, y_o, cp);
+                if (phase == 0) xs.cost[s][r * 64 + lane] = c;
+                else xs.cost_r[phase == 2 ? 1 : r][s][lane] = c;
+            }
+        }
+        __syncthreads();
+        // the end is one wave's; before it every wave goes on for itself (each
+        // needs the hypothesis that the next draw starts from)
+        const bool last = phase == 2 || (phase == 1 && both);
+        if (last && wave != 0) return;
+        if (active) {
+            if (phase == 0) {
+#pragma unroll 1
+                for (int k = 0; k < 4; ++k) {
+                    if (!((need >> k) & 1u)) continue;
+                    const float c = split_mean(v, xs.cost, base++);
+                    if (c < bc) { bc = c; best = xs.hyp[lane | (k << 6)]; changed = true; }
+                }
+            } else {
+                int second = 1;   // where the second step's costs are
+                if (phase == 1) {
+                    const float c = split_mean(v, xs.cost_r[0], lane);
+                    if (c < bc) { bc = c; best = draw(0, best); changed = true; second = 2; }
+                }
+                if (last) {
+                    const float c = split_mean(v, xs.cost_r[phase == 2 ? 1 : second], lane);
+                    if (c < bc) { bc = c; best = draw(1, best); changed = true; }
+                }
+            }
+        }
+        if (last) break;
+    }
+    if (!active) return;
+    v.hyp[parity][p] = best;
+    v.cost[parity][p] = bc;
+    v.chg[parity][p] = changed ? 1 : 0;
+}
+
+// The initial cost likewise: a wave per source.
+template <int NT, int ST, int STORE, int TX, int TY>
+__device__ __forceinline__ void cost_split(const DevView& v, float* tile, int bx, int by,
+                                           int parity, SplitXchg& xs)
+{
+    static_assert(TX * TY == 64, "one wave of pixels per tile");
+    constexpr int R = (NT - 1) * ST / 2;
+    using G = TileGeom<R, STORE, TX, TY>;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int waves = (int)blockDim.x >> 6;
+    const int tx = lane % TX, ty = lane / TX;
+    const int i = bx * TX + tx, y = by * TY + ty;
+    const int x = 2 * i + ((y + parity) & 1);
+    const bool active = y < v.H && x < v.W;
+    stage_ref_tile<R, STORE, TX, TY>(v, tile, bx, by, (int)blockDim.x);
+    if (active) {
+        const float4 h = v.hyp[parity][y * v.Wc + i];
+        const float* lwin = tile + ty * G::LP + (x - 2 * bx * TX);
+        const WinRef wr = window_ref_sums<NT, ST>(lwin, G::LP);
+        double rx, ry, rz;
+        ray_fp64(v.kinv_d, x, y, rx, ry, rz);
+        CandPlane cp;
+        const bool ok = cand_plane(v, x, y, rx, ry, rz, h.x, h.y, h.z, h.w, cp);
+#pragma unroll 1
+        for (int s = wave; s < v.S; s += waves) {
+            float c = 2.0f;
+            if (ok) c = source_cost<NT, ST, STORE, kCostChunk<NT>>(v, s, lwin, G::LP, wr, x, y, cp);
+            xs.cost[s][lane] = c;
+        }
+    }
+    __syncthreads();
+    if (wave == 0 && active) v.cost[parity][y * v.Wc + i] = split_mean(v, xs.cost, lane);
 }
 
 // Row-major outputs of pixel (x, y) from the colour planes.

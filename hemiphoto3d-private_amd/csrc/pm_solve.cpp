@@ -1,6 +1,6 @@
 // pm_solve.cpp -- per-view launch sequence (patchmatch_mvs.cu:1093-1258).
 //
-// init -> cost(red) -> cost(black) -> iterations x {half-pass red, black}
+// init -> cost -> iterations x {half-pass red, black}
 // -> finalize, all on the context stream, one synchronisation at the end.
 #include <algorithm>
 #include <cstring>
@@ -136,8 +136,7 @@ int enqueue_passes(hp3d_pm_ctx* ctx, const hp3d_view_desc* d, const Image* ref, 
     rc = apply_seeds(ctx, v, d);
     if (rc) return rc;
     ctx->mark(kPhaseInit);
-    for (int parity = 0; parity < 2 && e == hipSuccess; ++parity)
-        e = launch_pass(v, ref->store, d->radius, d->stride, kPassCost, 0, parity, 0, ctx->stream);
+    e = launch_pass(v, ref->store, d->radius, d->stride, kPassCost, 0, 0, 0, ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "cost launch");
     ctx->mark(kPhaseCost);
     for (int it = d->first_iteration; it < d->first_iteration + d->iterations; ++it)
@@ -333,9 +332,7 @@ int cost_only(hp3d_pm_ctx* ctx, const hp3d_view_desc* d, const Image* ref,
     if (rc) return rc;
     rc = import_hypotheses(ctx, v, depth, normal);
     if (rc) return rc;
-    hipError_t e = hipSuccess;
-    for (int parity = 0; parity < 2 && e == hipSuccess; ++parity)
-        e = launch_pass(v, ref->store, d->radius, d->stride, kPassCost, 0, parity, 0, ctx->stream);
+    hipError_t e = launch_pass(v, ref->store, d->radius, d->stride, kPassCost, 0, 0, 0, ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "cost launch");
     rc = emit_outputs(ctx, v, nullptr, nullptr, cost, nullptr, false);
     if (rc) return rc;

@@ -12,12 +12,18 @@
 namespace hp3d {
 
 // The grid must be 1-D with a multiple of 8 blocks.  Returns false for the
-// padding blocks past the last tile.
-__device__ __forceinline__ bool xcd_tile(int tiles_x, int tiles, int& bx, int& by)
+// padding blocks past the last of `n` units.
+__device__ __forceinline__ bool xcd_unit(int n, int& t)
 {
     const int nb = gridDim.x, b = blockIdx.x;
-    const int t = (b & 7) * (nb >> 3) + (b >> 3);
-    if (t >= tiles) return false;
+    t = (b & 7) * (nb >> 3) + (b >> 3);
+    return t < n;
+}
+
+__device__ __forceinline__ bool xcd_tile(int tiles_x, int tiles, int& bx, int& by)
+{
+    int t;
+    if (!xcd_unit(tiles, t)) return false;
     by = t / tiles_x;
     bx = t - by * tiles_x;
     return true;
