@@ -429,10 +429,10 @@ class Context:
 
     def run_view(self, desc, shape, with_normal=True, with_cost=True, with_confidence=False):
         H, W = shape
-        depth = np.zeros((H, W), dtype=np.float32)
-        normal = np.zeros((H, W, 3), dtype=np.float32) if with_normal else None
-        cost = np.zeros((H, W), dtype=np.float32) if with_cost else None
-        conf = np.zeros((H, W), dtype=np.float32) if with_confidence else None
+        depth = np.empty((H, W), dtype=np.float32)
+        normal = np.empty((H, W, 3), dtype=np.float32) if with_normal else None
+        cost = np.empty((H, W), dtype=np.float32) if with_cost else None
+        conf = np.empty((H, W), dtype=np.float32) if with_confidence else None
         out = ViewOut(_p(depth, _f32p), _p(normal, _f32p) if with_normal else None,
                       _p(cost, _f32p) if with_cost else None,
                       _p(conf, _f32p) if with_confidence else None, 0)
@@ -513,9 +513,9 @@ class Context:
         outs = (ViewOut * n)()
         res = []
         for j, (H, W) in enumerate(shapes):
-            r = {"depth": np.zeros((H, W), np.float32),
-                 "normal": np.zeros((H, W, 3), np.float32) if with_normal else None,
-                 "cost": np.zeros((H, W), np.float32) if with_cost else None}
+            r = {"depth": np.empty((H, W), np.float32),
+                 "normal": np.empty((H, W, 3), np.float32) if with_normal else None,
+                 "cost": np.empty((H, W), np.float32) if with_cost else None}
             outs[j] = ViewOut(_p(r["depth"], _f32p),
                               _p(r["normal"], _f32p) if with_normal else None,
                               _p(r["cost"], _f32p) if with_cost else None, None, 0)
@@ -595,9 +595,9 @@ class Context:
         _check(lib().hp3d_pm_fuse(self.h, arr, n, float(min_confidence), None, None, None, 0,
                                   ctypes.byref(cnt)), self.h)
         N = cnt.value
-        pos = np.zeros((N, 3), np.float32)
-        nrm = np.zeros((N, 3), np.float32) if with_normals else None
-        col = np.zeros((N, 3), np.float32) if with_colors else None
+        pos = np.empty((N, 3), np.float32)
+        nrm = np.empty((N, 3), np.float32) if with_normals else None
+        col = np.empty((N, 3), np.float32) if with_colors else None
         if N:
             _check(lib().hp3d_pm_fuse(self.h, arr, n, float(min_confidence), _p(pos, _f32p),
                                       _p(nrm, _f32p) if with_normals else None,
@@ -622,8 +622,8 @@ class Context:
 
     def init_hypotheses(self, desc, shape):
         H, W = shape
-        depth = np.zeros((H, W), dtype=np.float32)
-        normal = np.zeros((H, W, 3), dtype=np.float32)
+        depth = np.empty((H, W), dtype=np.float32)
+        normal = np.empty((H, W, 3), dtype=np.float32)
         _check(lib().hp3d_pm_init_hypotheses(self.h, ctypes.byref(desc), _p(depth, _f32p),
                                              _p(normal, _f32p)), self.h)
         return depth, normal
@@ -631,7 +631,7 @@ class Context:
     def cost_eval(self, desc, depth, normal):
         depth = np.ascontiguousarray(depth, dtype=np.float32)
         normal = np.ascontiguousarray(normal, dtype=np.float32)
-        cost = np.zeros(depth.shape, dtype=np.float32)
+        cost = np.empty(depth.shape, dtype=np.float32)
         _check(lib().hp3d_pm_cost_eval(self.h, ctypes.byref(desc), _p(depth, _f32p),
                                        _p(normal, _f32p), _p(cost, _f32p)), self.h)
         return cost

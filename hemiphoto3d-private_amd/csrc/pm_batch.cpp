@@ -381,16 +381,15 @@ int hp3d_pm_batch_run(hp3d_pm_ctx* ctx, const hp3d_view_desc* descs, int n,
     }
     if (e != hipSuccess) return ctx->hip_fail(e, "batch launch");
     ctx->mark(kPhasePropagate);
-    for (int j = 0; j < n && e == hipSuccess; ++j) {
+    for (int j = 0; j < n && e == hipSuccess; ++j) {   // view by view, in order
         if (outs[j].on_device) continue;
-        const size_t px = (size_t)jobs[j].v.W * jobs[j].v.H;
-        struct { float* dst; const float* src; size_t count; } cp[4] = {
-            {outs[j].depth, jobs[j].out_depth, px}, {outs[j].normal, jobs[j].out_normal, 3 * px},
-            {outs[j].cost, jobs[j].out_cost, px}, {outs[j].confidence, jobs[j].out_conf, px}};
-        for (auto& c : cp)
-            if (c.dst && e == hipSuccess)
-                e = hipMemcpyAsync(c.dst, c.src, c.count * sizeof(float), hipMemcpyDeviceToHost,
-                                   ctx->stream);
+        const size_t px = (size_t)jobs[j].v.W * jobs[j].v.H * sizeof(float);
+        std::vector<HostLink::Seg> segs;
+        if (outs[j].depth) segs.push_back({outs[j].depth, jobs[j].out_depth, px});
+        if (outs[j].normal) segs.push_back({outs[j].normal, jobs[j].out_normal, 3 * px});
+        if (outs[j].cost) segs.push_back({outs[j].cost, jobs[j].out_cost, px});
+        if (outs[j].confidence) segs.push_back({outs[j].confidence, jobs[j].out_conf, px});
+        e = ctx->link.download(segs, ctx->stream);
     }
     if (e != hipSuccess) return ctx->hip_fail(e, "batch output copy");
     ctx->mark(kPhaseFinalize);

@@ -330,7 +330,7 @@ int hp3d_pm_image_upload(hp3d_pm_ctx* ctx, const void* data, int W, int H, size_
     rc = ctx->grow(ctx->staging, stage_bytes, "upload staging");
     if (rc) { release(); return rc; }
     void* stage = ctx->staging.ptr;
-    hipError_t e = hipMemcpyAsync(stage, data, stage_bytes, hipMemcpyHostToDevice, ctx->stream);
+    hipError_t e = ctx->link.upload({{const_cast<void*>(data), stage, stage_bytes}}, ctx->stream);
     if (e == hipSuccess)
         e = launch_img_prep(fmt == HP3D_FMT_U8 ? (const uint8_t*)stage : nullptr,
                             fmt == HP3D_FMT_F32 ? (const float*)stage : nullptr, pitch, W, H,
@@ -541,10 +541,11 @@ int hp3d_pm_device_copy(hp3d_pm_ctx* ctx, void* dst, const void* src, size_t byt
     if (!ctx) return HP3D_ERR_INVALID_ARG;
     if (!dst || !src || kind < 0 || kind > 2)
         return ctx->fail(HP3D_ERR_INVALID_ARG, "device_copy: bad arguments");
-    static const hipMemcpyKind kinds[3] = {hipMemcpyHostToDevice, hipMemcpyDeviceToHost,
-                                           hipMemcpyDeviceToDevice};
     (void)hipSetDevice(ctx->device);
-    hipError_t e = hipMemcpyAsync(dst, src, bytes, kinds[kind], ctx->stream);
+    hipError_t e;
+    if (kind == 0) e = ctx->link.upload({{const_cast<void*>(src), dst, bytes}}, ctx->stream);
+    else if (kind == 1) e = ctx->link.download({{dst, const_cast<void*>(src), bytes}}, ctx->stream);
+    else e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     return e == hipSuccess ? HP3D_OK : ctx->hip_fail(e, "device_copy");
 }

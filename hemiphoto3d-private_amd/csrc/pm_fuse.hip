@@ -194,8 +194,8 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
     long long* d_total = reinterpret_cast<long long*>(base + scan_off + a256(max_blocks * 4) +
                                                       a256(max_blocks * 8));
     std::vector<FuseViewDev> g(n);
-    hipError_t e = hipSuccess;
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
+    std::vector<HostLink::Seg> segs;
+    for (int i = 0; i < n; ++i) {
         const hp3d_fuse_view& v = views[i];
         const size_t px = (size_t)v.width * v.height;
         char* p = base + off[i];
@@ -213,24 +213,24 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
         d.channels = v.color ? v.color_channels : 0;
         d.min_conf = min_confidence;
         d.depth = reinterpret_cast<float*>(p);
-        e = hipMemcpyAsync(p, v.depth, px * 4, hipMemcpyHostToDevice, ctx->stream);
+        segs.push_back({const_cast<float*>(v.depth), p, px * 4});
         p += a256(px * 4);
-        if (v.normal && e == hipSuccess) {
+        if (v.normal) {
             d.normal = reinterpret_cast<float*>(p);
-            e = hipMemcpyAsync(p, v.normal, px * 12, hipMemcpyHostToDevice, ctx->stream);
+            segs.push_back({const_cast<float*>(v.normal), p, px * 12});
             p += a256(px * 12);
         }
-        if (v.confidence && e == hipSuccess) {
+        if (v.confidence) {
             d.conf = reinterpret_cast<float*>(p);
-            e = hipMemcpyAsync(p, v.confidence, px * 4, hipMemcpyHostToDevice, ctx->stream);
+            segs.push_back({const_cast<float*>(v.confidence), p, px * 4});
             p += a256(px * 4);
         }
-        if (v.color && e == hipSuccess) {
+        if (v.color) {
             d.color = reinterpret_cast<uint8_t*>(p);
-            e = hipMemcpyAsync(p, v.color, px * v.color_channels, hipMemcpyHostToDevice,
-                               ctx->stream);
+            segs.push_back({const_cast<uint8_t*>(v.color), p, px * v.color_channels});
         }
     }
+    hipError_t e = ctx->link.upload(segs, ctx->stream);
     // pass 1: count every view, in order, to size the output
     std::vector<long long> view_base(n + 1, 0);
     for (int i = 0; i < n && e == hipSuccess; ++i) {
@@ -283,12 +283,10 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
                            d_offsets, d_pos, d_nrm, d_col);
         e = hipGetLastError();
     }
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(positions, d_pos, per, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess && normals)
-        e = hipMemcpyAsync(normals, d_nrm, per, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess && colors)
-        e = hipMemcpyAsync(colors, d_col, per, hipMemcpyDeviceToHost, ctx->stream);
+    segs.assign({{positions, d_pos, per}});
+    if (normals) segs.push_back({normals, d_nrm, per});
+    if (colors) segs.push_back({colors, d_col, per});
+    if (e == hipSuccess) e = ctx->link.download(segs, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     ctx->dev_free(out, per * nbuf);
     ctx->dev_free(block, total);

@@ -142,15 +142,14 @@ extern "C" int hp3d_pm_geom_filter(hp3d_pm_ctx* ctx, hp3d_geom_view* views, int 
         const size_t px = (size_t)views[i].width * views[i].height;
         return reinterpret_cast<float*>(static_cast<char*>(block) + off[i]) + (k == 4 ? 4 * px : k * px);
     };
-    hipError_t e = hipSuccess;
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
-        const size_t px = (size_t)views[i].width * views[i].height;
-        e = hipMemcpyAsync(dptr(i, 0), views[i].depth, px * 4, hipMemcpyHostToDevice, ctx->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(dptr(i, 1), views[i].normal, 3 * px * 4, hipMemcpyHostToDevice, ctx->stream);
-        if (e == hipSuccess && views[i].confidence)
-            e = hipMemcpyAsync(dptr(i, 4), views[i].confidence, px * 4, hipMemcpyHostToDevice, ctx->stream);
+    std::vector<HostLink::Seg> segs;
+    for (int i = 0; i < n; ++i) {
+        const size_t px = (size_t)views[i].width * views[i].height * 4;
+        segs.push_back({views[i].depth, dptr(i, 0), px});
+        segs.push_back({const_cast<float*>(views[i].normal), dptr(i, 1), 3 * px});
+        if (views[i].confidence) segs.push_back({views[i].confidence, dptr(i, 4), px});
     }
+    hipError_t e = ctx->link.upload(segs, ctx->stream);
     const float cos_tol = std::cos(normal_tol_deg * 3.14159265358979323846f / 180.0f);
     std::vector<char> filtered(n, 0);
     double ki[9];
@@ -189,11 +188,11 @@ extern "C" int hp3d_pm_geom_filter(hp3d_pm_ctx* ctx, hp3d_geom_view* views, int 
         e = hipGetLastError();
         filtered[i] = 1;
     }
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
-        const size_t px = (size_t)views[i].width * views[i].height;
-        e = hipMemcpyAsync(views[i].depth, dptr(i, 0), px * 4, hipMemcpyDeviceToHost, ctx->stream);
-        if (e == hipSuccess && views[i].confidence)
-            e = hipMemcpyAsync(views[i].confidence, dptr(i, 4), px * 4, hipMemcpyDeviceToHost, ctx->stream);
+    for (int i = 0; i < n && e == hipSuccess; ++i) {   // view by view, in order
+        const size_t px = (size_t)views[i].width * views[i].height * 4;
+        segs.assign({{views[i].depth, dptr(i, 0), px}});
+        if (views[i].confidence) segs.push_back({views[i].confidence, dptr(i, 4), px});
+        e = ctx->link.download(segs, ctx->stream);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     ctx->dev_free(block, total);

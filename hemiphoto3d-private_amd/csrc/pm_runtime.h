@@ -10,6 +10,7 @@
 #include "../../include/hp3d_pm.h"
 #include "pm_device.h"
 #include "pm_launch.h"
+#include "pm_xfer.h"
 
 namespace hp3d {
 
@@ -78,7 +79,7 @@ struct hp3d_pm_ctx {
     hipEvent_t ev_fin[2] = {nullptr, nullptr}, ev_copied[2] = {nullptr, nullptr};
 
     // per-view working set, grown on demand and reused across views
-    hp3d::DevBuf hyp, cost, chg, out_depth, out_normal, out_cost, in_depth, in_normal, staging;
+    hp3d::DevBuf hyp, cost, chg, out_stage, in_hyp, staging;
     hp3d::DevBuf seed_pts, seed_owner;
 
     // batched form: state arena, job table, step items, captured graph
@@ -86,6 +87,8 @@ struct hp3d_pm_ctx {
     hipGraphExec_t batch_graph = nullptr;
     std::vector<unsigned char> batch_graph_key;
     std::map<int, int> tuned;   // (radius, stride, store) key -> variant
+
+    hp3d::HostLink link;   // copies to and from pageable host memory
 
     hp3d_pm_stats stats{};
     std::vector<hp3d::Mark> marks;
@@ -107,6 +110,7 @@ struct hp3d_pm_ctx {
     }
     void release_all()
     {
+        link.close();
         for (auto& kv : images) {
             dev_free(kv.second.plain, kv.second.plain_bytes);
             dev_free(kv.second.coef, kv.second.coef_bytes);
@@ -131,9 +135,8 @@ struct hp3d_pm_ctx {
             (void)hipGraphExecDestroy(batch_graph);
             batch_graph = nullptr;
         }
-        for (hp3d::DevBuf* b : {&hyp, &cost, &chg, &out_depth, &out_normal, &out_cost, &in_depth,
-                                &in_normal, &staging, &seed_pts, &seed_owner, &batch_state,
-                                &batch_jobs, &batch_items, &batch_done})
+        for (hp3d::DevBuf* b : {&hyp, &cost, &chg, &out_stage, &in_hyp, &staging, &seed_pts,
+                                &seed_owner, &batch_state, &batch_jobs, &batch_items, &batch_done})
             release_buf(*b);
     }
 };

@@ -147,6 +147,7 @@ struct hp3d_pm_server {
     uint64_t next_id = 0, next_image = 0;
     bool stop = false, comp_stop = false;
     std::thread thr, comp_thr;
+    HostLink link;                       // the completion thread's downloads
     hp3d_server_stats stats{};
     Clock::time_point t0;
     std::string last_error;
@@ -472,14 +473,11 @@ void hp3d_pm_server::complete_loop()
             completing.pop_front();
         }
         hipError_t e = hipEventSynchronize(j->last_ev);
-        const size_t px = (size_t)j->d.width * j->d.height;
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(j->d.out_depth, j->dj.out_depth, px * 4, hipMemcpyDeviceToHost, copy);
-        if (e == hipSuccess && j->d.out_normal)
-            e = hipMemcpyAsync(j->d.out_normal, j->dj.out_normal, 3 * px * 4,
-                               hipMemcpyDeviceToHost, copy);
-        if (e == hipSuccess && j->d.out_cost)
-            e = hipMemcpyAsync(j->d.out_cost, j->dj.out_cost, px * 4, hipMemcpyDeviceToHost, copy);
+        const size_t px = (size_t)j->d.width * j->d.height * 4;
+        std::vector<HostLink::Seg> segs{{j->d.out_depth, j->dj.out_depth, px}};
+        if (j->d.out_normal) segs.push_back({j->d.out_normal, j->dj.out_normal, 3 * px});
+        if (j->d.out_cost) segs.push_back({j->d.out_cost, j->dj.out_cost, px});
+        if (e == hipSuccess) e = link.download(segs, copy);
         if (e == hipSuccess) e = hipStreamSynchronize(copy);
         std::lock_guard<std::mutex> lk(mu);
         if (e != hipSuccess) last_error = hipGetErrorString(e);
@@ -822,6 +820,7 @@ int hp3d_server_destroy(hp3d_pm_server* s)
     }
     if (s->comp_thr.joinable()) s->comp_thr.join();
     (void)hipSetDevice(s->device);
+    s->link.close();
     for (hipStream_t st : {s->compute, s->upload, s->copy, s->image})
         if (st) (void)hipStreamSynchronize(st);
     {

@@ -37,18 +37,13 @@ int bind_state(hp3d_pm_ctx* ctx, DevView& v)
 int import_hypotheses(hp3d_pm_ctx* ctx, const DevView& v, const float* depth, const float* normal)
 {
     const size_t n = (size_t)v.W * v.H;
-    int rc = ctx->grow(ctx->in_depth, n * sizeof(float), "input depth");
+    int rc = ctx->grow(ctx->in_hyp, 4 * n * sizeof(float), "input hypotheses");
     if (rc) return rc;
-    rc = ctx->grow(ctx->in_normal, 3 * n * sizeof(float), "input normal");
-    if (rc) return rc;
-    hipError_t e = hipMemcpyAsync(ctx->in_depth.ptr, depth, n * sizeof(float),
-                                  hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(ctx->in_normal.ptr, normal, 3 * n * sizeof(float),
-                           hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess)
-        e = launch_import(v, (const float*)ctx->in_depth.ptr, (const float*)ctx->in_normal.ptr,
-                          ctx->stream);
+    float* d = static_cast<float*>(ctx->in_hyp.ptr);
+    hipError_t e = ctx->link.upload({{const_cast<float*>(depth), d, n * sizeof(float)},
+                                     {const_cast<float*>(normal), d + n, 3 * n * sizeof(float)}},
+                                    ctx->stream);
+    if (e == hipSuccess) e = launch_import(v, d, d + n, ctx->stream);
     return e == hipSuccess ? HP3D_OK : ctx->hip_fail(e, "hypothesis import");
 }
 
@@ -79,32 +74,24 @@ int emit_outputs(hp3d_pm_ctx* ctx, const DevView& v, float* depth, float* normal
         e = launch_finalize(v, depth, normal, cost, conf, ctx->stream);
         return e == hipSuccess ? HP3D_OK : ctx->hip_fail(e, "finalize");
     }
-    int rc = HP3D_OK;
-    float* dd = nullptr;
-    float* dn = nullptr;
-    float* dc = nullptr;
-    if (depth) {
-        rc = ctx->grow(ctx->out_depth, n * sizeof(float), "output depth");
-        dd = static_cast<float*>(ctx->out_depth.ptr);
-    }
-    if (!rc && normal) {
-        rc = ctx->grow(ctx->out_normal, 3 * n * sizeof(float), "output normal");
-        dn = static_cast<float*>(ctx->out_normal.ptr);
-    }
-    if (!rc && (cost || conf)) {
-        rc = ctx->grow(ctx->out_cost, 2 * n * sizeof(float), "output cost");
-        dc = static_cast<float*>(ctx->out_cost.ptr);
-    }
+    // staged side by side, so that a small view's maps come over in one copy
+    float* const host[4] = {depth, normal, cost, conf};
+    const size_t count[4] = {n, 3 * n, n, n};
+    float* dev[4] = {};
+    size_t total = 0;
+    for (int q = 0; q < 4; ++q) total += host[q] ? count[q] : 0;
+    int rc = ctx->grow(ctx->out_stage, total * sizeof(float), "output staging");
     if (rc) return rc;
-    e = launch_finalize(v, dd, dn, cost ? dc : nullptr, conf ? dc + n : nullptr, ctx->stream);
-    if (e == hipSuccess && depth)
-        e = hipMemcpyAsync(depth, dd, n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess && normal)
-        e = hipMemcpyAsync(normal, dn, 3 * n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess && cost)
-        e = hipMemcpyAsync(cost, dc, n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess && conf)
-        e = hipMemcpyAsync(conf, dc + n, n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream);
+    std::vector<HostLink::Seg> segs;
+    float* p = static_cast<float*>(ctx->out_stage.ptr);
+    for (int q = 0; q < 4; ++q) {
+        if (!host[q]) continue;
+        dev[q] = p;
+        segs.push_back({host[q], p, count[q] * sizeof(float)});
+        p += count[q];
+    }
+    e = launch_finalize(v, dev[0], dev[1], dev[2], dev[3], ctx->stream);
+    if (e == hipSuccess) e = ctx->link.download(segs, ctx->stream);
     return e == hipSuccess ? HP3D_OK : ctx->hip_fail(e, "output copy");
 }
 
@@ -233,8 +220,7 @@ int solve_views(hp3d_pm_ctx* ctx, int n, const hp3d_view_desc* d, const Image* c
                 seed_px = std::max(seed_px, px);
             }
         }
-        if (in_px) rc = ctx->grow(ctx->in_depth, in_px * sizeof(float), "input depth");
-        if (!rc && in_px) rc = ctx->grow(ctx->in_normal, 3 * in_px * sizeof(float), "input normal");
+        if (in_px) rc = ctx->grow(ctx->in_hyp, 4 * in_px * sizeof(float), "input hypotheses");
         if (!rc && seed_bytes) rc = ctx->grow(ctx->seed_pts, seed_bytes, "seed points");
         if (!rc && seed_px) rc = ctx->grow(ctx->seed_owner, seed_px * sizeof(int), "seed owner map");
         if (rc) return rc;
@@ -289,10 +275,10 @@ int solve_views(hp3d_pm_ctx* ctx, int n, const hp3d_view_desc* d, const Image* c
             float* dst[4] = {out[j].depth, out[j].normal, out[j].cost, out[j].confidence};
             const size_t cnt[4] = {px, 3 * px, px, px};
             e = hipStreamWaitEvent(ctx->copy_stream, ctx->ev_fin[k], 0);
-            for (int q = 0; q < 4 && e == hipSuccess; ++q)
-                if (dst[q])
-                    e = hipMemcpyAsync(dst[q], sd[k][q], cnt[q] * sizeof(float),
-                                       hipMemcpyDeviceToHost, ctx->copy_stream);
+            std::vector<HostLink::Seg> segs;
+            for (int q = 0; q < 4; ++q)
+                if (dst[q]) segs.push_back({dst[q], sd[k][q], cnt[q] * sizeof(float)});
+            if (e == hipSuccess) e = ctx->link.download(segs, ctx->copy_stream);
             if (e == hipSuccess) e = hipEventRecord(ctx->ev_copied[k], ctx->copy_stream);
             if (e != hipSuccess) rc = ctx->hip_fail(e, "output download");
         }

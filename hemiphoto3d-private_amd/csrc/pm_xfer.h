@@ -1,0 +1,101 @@
+// pm_xfer.h -- copies between pageable host memory and the device.
+//
+// The runtime's own copy of pageable memory stages it through one thread: 17
+// GB/s to the host, 36 GB/s from it, and 60 us for a small view's maps, against
+// 57 GB/s and 11 us from page-locked memory; a caller's fresh arrays, whose
+// pages are touched for the first time, take 4 to 14 GB/s a thread.  A HostLink
+// keeps a ring of page-locked slots: the link fills or drains them in order on
+// a stream while a few threads copy between the slots and the caller's memory,
+// or, for copies of up to a few slots, the calling thread alone.  Page-locked
+// host memory is copied by the link directly.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <atomic>
+#include <condition_variable>
+#include <cstddef>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace hp3d {
+
+// One host thread at a time.  Ring and threads are made by the first copy that
+// needs them and given back by close().
+class HostLink {
+public:
+    // `bytes` of host memory and of device memory.  Neighbouring segments that
+    // are adjacent on the device share slots.
+    struct Seg {
+        void* host;
+        void* dev;
+        size_t bytes;
+    };
+
+    HostLink() = default;
+    HostLink(const HostLink&) = delete;
+    HostLink& operator=(const HostLink&) = delete;
+    ~HostLink() { close(); }
+
+    // (The order in which the parts of one call are written is not defined.)
+    // Device to host, after the work queued on st.  Returns when pageable
+    // destinations are written; page-locked ones are once st is synchronised.
+    hipError_t download(const std::vector<Seg>& segs, hipStream_t st);
+    // Host to device on st.  Returns when pageable sources are read; page-locked
+    // ones are once st is synchronised.
+    hipError_t upload(const std::vector<Seg>& segs, hipStream_t st);
+    // Waits for the ring's copies and gives everything back.
+    void close();
+
+private:
+    // 2 MiB a copy of the link (57 GB/s less 5 us each) where there are many,
+    // 1 MiB below, so that the threads start early; a copy of up to 3 pieces is
+    // over before threads have woken
+    static constexpr int kSlots = 8;
+    static constexpr size_t kSlotBytes = 2u << 20;
+    static constexpr size_t kSmallBytes = 1u << 20;
+    static constexpr size_t kManyBytes = 16u << 20;
+    static constexpr size_t kAlonePieces = 3;
+    static constexpr int kTasks = 4;       // a piece's shares among the threads
+    static constexpr int kMaxParts = 4;
+    static constexpr int kMaxWorkers = 6;
+
+    struct Piece {   // one slot's worth: adjacent device memory, its host parts
+        char* dev = nullptr;
+        size_t bytes = 0;
+        int parts = 0;
+        struct { char* host; size_t off, bytes; } part[kMaxParts];
+    };
+
+    bool open();
+    void start_workers();
+    hipError_t split(const std::vector<Seg>& segs, bool to_host, hipStream_t st);
+    hipError_t plain(bool to_host, hipStream_t st);
+    void copy_task(size_t i);
+    bool work_one();
+    void worker();
+    void begin(bool to_host);
+    void wake();
+    void hand_out(size_t piece);
+    void end();
+    hipError_t slot_ready(int slot);
+    char* slot_ptr(size_t piece) { return ring_ + (piece % kSlots) * kSlotBytes; }
+
+    char* ring_ = nullptr;
+    hipEvent_t ev_[kSlots] = {};
+    bool in_flight_[kSlots] = {};   // ev_ of a copy out of the slot, not waited for yet
+    std::vector<Piece> pieces_;
+    std::atomic<int> left_[kSlots] = {};   // tasks of the slot's piece not done yet
+
+    // the copy the threads are at: tasks [0, ready_) may be taken
+    bool to_host_ = false;
+    std::atomic<size_t> ready_{0}, taken_{0};
+    std::atomic<bool> active_{false};
+    std::mutex mu_;
+    std::condition_variable cv_;
+    bool stop_ = false;
+    int inside_ = 0;                // workers in the copy (mu_)
+    std::vector<std::thread> workers_;
+};
+
+}  // namespace hp3d
