@@ -381,16 +381,16 @@ int hp3d_pm_batch_run(hp3d_pm_ctx* ctx, const hp3d_view_desc* descs, int n,
     }
     if (e != hipSuccess) return ctx->hip_fail(e, "batch launch");
     ctx->mark(kPhasePropagate);
-    for (int j = 0; j < n && e == hipSuccess; ++j) {   // view by view, in order
+    std::vector<HostLink::Seg> segs;
+    for (int j = 0; j < n; ++j) {
         if (outs[j].on_device) continue;
         const size_t px = (size_t)jobs[j].v.W * jobs[j].v.H * sizeof(float);
-        std::vector<HostLink::Seg> segs;
         if (outs[j].depth) segs.push_back({outs[j].depth, jobs[j].out_depth, px});
         if (outs[j].normal) segs.push_back({outs[j].normal, jobs[j].out_normal, 3 * px});
         if (outs[j].cost) segs.push_back({outs[j].cost, jobs[j].out_cost, px});
         if (outs[j].confidence) segs.push_back({outs[j].confidence, jobs[j].out_conf, px});
-        e = ctx->link.download(segs, ctx->stream);
     }
+    e = ctx->link.download(segs, ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "batch output copy");
     ctx->mark(kPhaseFinalize);
     int ctl[kCtlWords] = {0, 0};

@@ -188,12 +188,13 @@ extern "C" int hp3d_pm_geom_filter(hp3d_pm_ctx* ctx, hp3d_geom_view* views, int 
         e = hipGetLastError();
         filtered[i] = 1;
     }
-    for (int i = 0; i < n && e == hipSuccess; ++i) {   // view by view, in order
+    segs.clear();
+    for (int i = 0; i < n; ++i) {
         const size_t px = (size_t)views[i].width * views[i].height * 4;
-        segs.assign({{views[i].depth, dptr(i, 0), px}});
+        segs.push_back({views[i].depth, dptr(i, 0), px});
         if (views[i].confidence) segs.push_back({views[i].confidence, dptr(i, 4), px});
-        e = ctx->link.download(segs, ctx->stream);
     }
+    if (e == hipSuccess) e = ctx->link.download(segs, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     ctx->dev_free(block, total);
     if (e != hipSuccess) return ctx->hip_fail(e, "geometric filter");

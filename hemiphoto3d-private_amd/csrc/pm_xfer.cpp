@@ -5,6 +5,7 @@
 #include <cstring>
 #include <new>
 #include <system_error>
+#include <utility>
 
 namespace hp3d {
 
@@ -20,6 +21,17 @@ bool known_to_runtime(const void* p)
         return false;
     }
     return a.type != hipMemoryTypeUnregistered;
+}
+
+bool overlap(const std::vector<HostLink::Seg>& segs)
+{
+    if (segs.size() < 2) return false;
+    std::vector<std::pair<const char*, size_t>> r;
+    for (const auto& s : segs) r.emplace_back(static_cast<const char*>(s.host), s.bytes);
+    std::sort(r.begin(), r.end());
+    for (size_t i = 1; i < r.size(); ++i)
+        if (r[i - 1].first + r[i - 1].second > r[i].first) return true;
+    return false;
 }
 
 }  // namespace
@@ -93,7 +105,8 @@ hipError_t HostLink::split(const std::vector<Seg>& segs, bool to_host, hipStream
             total += s.bytes;
         }
     }
-    const size_t chunk = total < kManyBytes ? kSmallBytes : kSlotBytes;
+    const size_t chunk = piece_bytes(total);
+    alone_ = total <= kAloneBytes;
     for (const Seg* s : mine) {
         char* host = static_cast<char*>(s->host);
         char* dev = static_cast<char*>(s->dev);
@@ -157,6 +170,13 @@ bool HostLink::work_one()
     return false;
 }
 
+// The calling thread while it waits: it copies until a worker has come; then
+// it only keeps the link busy.
+void HostLink::help()
+{
+    if (came_.load(std::memory_order_relaxed) || !work_one()) std::this_thread::yield();
+}
+
 void HostLink::worker()
 {
     std::unique_lock<std::mutex> lk(mu_);
@@ -165,6 +185,7 @@ void HostLink::worker()
         if (stop_) return;
         ++inside_;
         lk.unlock();
+        came_.store(true, std::memory_order_relaxed);
         // tasks come every few microseconds while a copy is on: no sleeping
         while (active_.load(std::memory_order_acquire))
             if (!work_one()) std::this_thread::yield();
@@ -177,6 +198,7 @@ void HostLink::worker()
 void HostLink::begin(bool to_host)
 {
     to_host_ = to_host;
+    came_.store(false, std::memory_order_relaxed);
     ready_.store(0, std::memory_order_relaxed);
     taken_.store(0, std::memory_order_relaxed);
 }
@@ -217,11 +239,16 @@ hipError_t HostLink::slot_ready(int slot)
 
 hipError_t HostLink::download(const std::vector<Seg>& segs, hipStream_t st)
 {
-    hipError_t e = split(segs, true, st);
+    hipError_t e = hipSuccess;
+    if (overlap(segs)) {
+        for (size_t i = 0; i < segs.size() && e == hipSuccess; ++i) e = download({segs[i]}, st);
+        return e;
+    }
+    e = split(segs, true, st);
     if (e != hipSuccess || pieces_.empty()) return e;
     const size_t n = pieces_.size();
     if (!open()) return plain(true, st);
-    if (n > kAlonePieces) start_workers();
+    if (!alone_) start_workers();
     begin(true);
     size_t issued = 0, handed = 0;
     while (handed < n && e == hipSuccess) {
@@ -239,7 +266,7 @@ hipError_t HostLink::download(const std::vector<Seg>& segs, hipStream_t st)
         }
         if (e != hipSuccess) break;
         if (issued == handed) {   // every slot is being emptied: help
-            if (!work_one()) std::this_thread::yield();
+            help();
             continue;
         }
         if (n == 1) {
@@ -247,12 +274,11 @@ hipError_t HostLink::download(const std::vector<Seg>& segs, hipStream_t st)
         } else if (handed == 0) {
             e = hipEventSynchronize(ev_[0]);   // the work before the copy, however long
         } else {
-            while ((e = hipEventQuery(ev_[handed % kSlots])) == hipErrorNotReady)
-                if (!work_one()) std::this_thread::yield();
+            while ((e = hipEventQuery(ev_[handed % kSlots])) == hipErrorNotReady) help();
         }
         if (e != hipSuccess) break;
         hand_out(handed++);
-        if (handed == 1 && n > kAlonePieces) wake();
+        if (handed == 1 && !alone_) wake();
     }
     (void)hipGetLastError();   // the queries' "not ready"
     end();
@@ -266,9 +292,9 @@ hipError_t HostLink::upload(const std::vector<Seg>& segs, hipStream_t st)
     if (e != hipSuccess || pieces_.empty()) return e;
     const size_t n = pieces_.size();
     if (!open()) return plain(false, st);
-    if (n > kAlonePieces) start_workers();
+    if (!alone_) start_workers();
     begin(false);
-    if (n > kAlonePieces) wake();
+    if (!alone_) wake();
     size_t handed = 0, issued = 0;
     while (issued < n && e == hipSuccess) {
         // without threads a piece at a time, so that the link starts early
@@ -279,8 +305,7 @@ hipError_t HostLink::upload(const std::vector<Seg>& segs, hipStream_t st)
         }
         if (e != hipSuccess) break;
         const int slot = (int)(issued % kSlots);
-        while (left_[slot].load(std::memory_order_acquire) > 0)
-            if (!work_one()) std::this_thread::yield();
+        while (left_[slot].load(std::memory_order_acquire) > 0) help();
         e = hipMemcpyAsync(pieces_[issued].dev, slot_ptr(issued), pieces_[issued].bytes,
                            hipMemcpyHostToDevice, st);
         if (e == hipSuccess) e = hipEventRecord(ev_[slot], st);

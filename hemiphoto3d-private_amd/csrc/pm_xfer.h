@@ -37,8 +37,8 @@ public:
     HostLink& operator=(const HostLink&) = delete;
     ~HostLink() { close(); }
 
-    // (The order in which the parts of one call are written is not defined.)
-    // Device to host, after the work queued on st.  Returns when pageable
+    // Device to host, after the work queued on st.  Where segments overlap in
+    // host memory the later one's bytes stay.  Returns when pageable
     // destinations are written; page-locked ones are once st is synchronised.
     hipError_t download(const std::vector<Seg>& segs, hipStream_t st);
     // Host to device on st.  Returns when pageable sources are read; page-locked
@@ -48,14 +48,17 @@ public:
     void close();
 
 private:
-    // 2 MiB a copy of the link (57 GB/s less 5 us each) where there are many,
-    // 1 MiB below, so that the threads start early; a copy of up to 3 pieces is
-    // over before threads have woken
+    // The link spends 10 to 15 us on each copy besides its bytes, so pieces are
+    // as large as still lets the threads work beside it (38 MB at 36 GB/s in
+    // pieces of 2 MiB, 42 in 4; 10 MB at 26 in 1 MiB, 31 in 2).  A copy of up to
+    // 3 MiB is over before threads have woken.
     static constexpr int kSlots = 8;
-    static constexpr size_t kSlotBytes = 2u << 20;
-    static constexpr size_t kSmallBytes = 1u << 20;
-    static constexpr size_t kManyBytes = 16u << 20;
-    static constexpr size_t kAlonePieces = 3;
+    static constexpr size_t kSlotBytes = 4u << 20;
+    static constexpr size_t kAloneBytes = 3u << 20;
+    static size_t piece_bytes(size_t total)
+    {
+        return total < (4u << 20) ? 1u << 20 : total < (24u << 20) ? 2u << 20 : kSlotBytes;
+    }
     static constexpr int kTasks = 4;       // a piece's shares among the threads
     static constexpr int kMaxParts = 4;
     static constexpr int kMaxWorkers = 6;
@@ -73,6 +76,7 @@ private:
     hipError_t plain(bool to_host, hipStream_t st);
     void copy_task(size_t i);
     bool work_one();
+    void help();
     void worker();
     void begin(bool to_host);
     void wake();
@@ -85,12 +89,13 @@ private:
     hipEvent_t ev_[kSlots] = {};
     bool in_flight_[kSlots] = {};   // ev_ of a copy out of the slot, not waited for yet
     std::vector<Piece> pieces_;
+    bool alone_ = true;             // no threads for this copy
     std::atomic<int> left_[kSlots] = {};   // tasks of the slot's piece not done yet
 
     // the copy the threads are at: tasks [0, ready_) may be taken
     bool to_host_ = false;
     std::atomic<size_t> ready_{0}, taken_{0};
-    std::atomic<bool> active_{false};
+    std::atomic<bool> active_{false}, came_{false};   // came_: a worker has
     std::mutex mu_;
     std::condition_variable cv_;
     bool stop_ = false;

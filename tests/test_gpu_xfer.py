@@ -65,3 +65,19 @@ def test_contexts_copy_at_once(pkg):
     for t in threads:
         t.join()
     assert not failed
+
+
+def test_overlapping_destinations_keep_the_later_output(pkg, ctx, scenes):
+    """Two views of a batch given one array: it holds the second view's map."""
+    job = scenes.plane_job(W=200, H=150, iterations=1)
+    hs = [ctx.upload(im) for im in [job.ref] + job.srcs]
+    descs = [pkg.make_desc(hs[0], hs[1:], job.Kinv, job.A, job.b, job.dmin, job.dmax, iterations=1,
+                           seed=s) for s in (1, 2)]
+    want = ctx.run_view(descs[1], job.shape)["depth"]
+    got = np.zeros(job.shape, np.float32)
+    outs = (pkg.ViewOut * 2)(*[pkg.ViewOut(pkg._p(got, pkg._f32p), None, None, None, 0)] * 2)
+    rc = pkg.lib().hp3d_pm_batch_run(ctx.h, (pkg.ViewDesc * 2)(*descs), 2, outs, None)
+    assert rc == 0
+    assert np.array_equal(got, want)
+    for h in hs:
+        ctx.release(h)
