@@ -9,9 +9,11 @@
 //   position = R^T (d K^-1 [x, y, 1] - t)   (world frame, include/types.h:55-74)
 //   normal   = R^T n                        (camera -> world)
 //   colour   = the pixel's 8-bit value / 255 (gray replicated, or RGB)
-// The maps are uploaded once; a count pass, a scan of the per-block counts
-// and a write pass place every point at its row-major rank, so the output is
-// deterministic.  Single-precision operations are written in one fixed order
+// A count pass over every view, one scan of the per-block counts and a write
+// pass place every point at its row-major rank, so the output is
+// deterministic; each pass is one launch over all views.  The maps come over
+// the link, which bounds the whole call: a call that only counts uploads depth
+// and confidence.  Single-precision operations are written in one fixed order
 // (no contraction), which the oracle restates.
 #include <hip/hip_runtime.h>
 
@@ -27,6 +29,10 @@ namespace hp3d {
 namespace {
 
 constexpr int kFuseBlock = 256;
+// Pixels of a workgroup, kFuseBlock at a time: an eighth of the counts to scan
+// (five 1280x960 views: count and scan 5 x 15 us in ten launches of 256-pixel
+// blocks, one launch each now).
+constexpr int kFuseSpan = 8 * kFuseBlock;
 
 struct FuseViewDev {
     float kinv[9], R[9], t[3];
@@ -36,6 +42,7 @@ struct FuseViewDev {
     const float* normal;
     const float* conf;
     const uint8_t* color;
+    int first_block;   // of the launch's blocks, in view order
 };
 
 __device__ __forceinline__ bool fuse_valid(const FuseViewDev& g, int q)
@@ -44,13 +51,30 @@ __device__ __forceinline__ bool fuse_valid(const FuseViewDev& g, int q)
     return d > 0.0f && (!g.conf || g.conf[q] >= g.min_conf);
 }
 
-__global__ __launch_bounds__(kFuseBlock) void fuse_count_kernel(FuseViewDev g, int* counts)
+// The view of this block: the last with first_block <= blockIdx.x.
+__device__ __forceinline__ const FuseViewDev& fuse_view(const FuseViewDev* views, int n)
 {
-    const int q = blockIdx.x * kFuseBlock + threadIdx.x;
-    const bool v = q < g.W * g.H && fuse_valid(g, q);
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (views[mid].first_block <= (int)blockIdx.x) lo = mid;
+        else hi = mid - 1;
+    }
+    return views[lo];
+}
+
+__global__ __launch_bounds__(kFuseBlock) void fuse_count_kernel(const FuseViewDev* views, int n,
+                                                                int* counts)
+{
+    const FuseViewDev& g = fuse_view(views, n);
+    const long long q0 = (long long)((int)blockIdx.x - g.first_block) * kFuseSpan + threadIdx.x;
+    const long long px = (long long)g.W * g.H;
     __shared__ int part[kFuseBlock / 64];
-    const unsigned long long m = __ballot(v);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = __popcll(m);
+    int c = 0;
+#pragma unroll
+    for (int k = 0; k < kFuseSpan; k += kFuseBlock)
+        c += __popcll(__ballot(q0 + k < px && fuse_valid(g, (int)(q0 + k))));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = c;
     __syncthreads();
     if (threadIdx.x == 0) {
         int s = 0;
@@ -59,14 +83,14 @@ __global__ __launch_bounds__(kFuseBlock) void fuse_count_kernel(FuseViewDev g, i
     }
 }
 
-// Exclusive scan of n block counts in place (one workgroup; n is at most a
-// few hundred thousand), total into *total.
-__global__ __launch_bounds__(1024) void fuse_scan_kernel(int* counts, int n, long long base,
+// Exclusive scan of n block counts (one workgroup; n is at most a few hundred
+// thousand), total into *total.
+__global__ __launch_bounds__(1024) void fuse_scan_kernel(const int* counts, int n,
                                                          long long* offsets, long long* total)
 {
     __shared__ long long carry;
     __shared__ long long part[1024 / 64];
-    if (threadIdx.x == 0) carry = base;
+    if (threadIdx.x == 0) carry = 0;
     __syncthreads();
     for (int start = 0; start < n; start += 1024) {
         const int i = start + threadIdx.x;
@@ -97,21 +121,10 @@ __global__ __launch_bounds__(1024) void fuse_scan_kernel(int* counts, int n, lon
     if (threadIdx.x == 0) *total = carry;
 }
 
-__global__ __launch_bounds__(kFuseBlock) void fuse_write_kernel(FuseViewDev g,
-                                                                const long long* offsets,
-                                                                float* pos, float* nrm, float* col)
+// The point of pixel q, written at rank o.
+__device__ __forceinline__ void fuse_point(const FuseViewDev& g, int q, long long o, float* pos,
+                                           float* nrm, float* col)
 {
-    const int q = blockIdx.x * kFuseBlock + threadIdx.x;
-    const bool v = q < g.W * g.H && fuse_valid(g, q);
-    __shared__ int part[kFuseBlock / 64];
-    const unsigned long long m = __ballot(v);
-    const int lane = threadIdx.x & 63;
-    if (lane == 0) part[threadIdx.x >> 6] = __popcll(m);
-    __syncthreads();
-    if (!v) return;
-    int rank = __popcll(m & ((1ull << lane) - 1ull));
-    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) rank += part[w];
-    const long long o = offsets[blockIdx.x] + rank;
     const int y = q / g.W, x = q - y * g.W;
     const float d = g.depth[q];
     const float fx = (float)x, fy = (float)y;
@@ -150,6 +163,35 @@ __global__ __launch_bounds__(kFuseBlock) void fuse_write_kernel(FuseViewDev g,
     }
 }
 
+__global__ __launch_bounds__(kFuseBlock) void fuse_write_kernel(const FuseViewDev* views, int n,
+                                                                const long long* offsets,
+                                                                float* pos, float* nrm, float* col)
+{
+    const FuseViewDev& g = fuse_view(views, n);
+    const long long q0 = (long long)((int)blockIdx.x - g.first_block) * kFuseSpan + threadIdx.x;
+    const long long px = (long long)g.W * g.H;
+    __shared__ int part[2][kFuseBlock / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    long long base = offsets[blockIdx.x];
+    for (int k = 0; k < kFuseSpan / kFuseBlock; ++k) {
+        const long long q = q0 + k * kFuseBlock;
+        const bool v = q < px && fuse_valid(g, (int)q);
+        const unsigned long long m = __ballot(v);
+        // (two sets: the next row's counts are written while this one's are read)
+        if (lane == 0) part[k & 1][wave] = __popcll(m);
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int w = 0; w < kFuseBlock / 64; ++w) {
+            if (w < wave) before += part[k & 1][w];
+            all += part[k & 1][w];
+        }
+        if (v)
+            fuse_point(g, (int)q, base + before + __popcll(m & ((1ull << lane) - 1ull)), pos, nrm,
+                       col);
+        base += all;
+    }
+}
+
 }  // namespace
 
 }  // namespace hp3d
@@ -171,86 +213,80 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
             return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: view %d is malformed", i);
     }
     (void)hipSetDevice(ctx->device);
-    // one device block per call: maps of every view, block counts, offsets
-    std::vector<size_t> off(n);
-    size_t total = 0, max_blocks = 0;
+    // what the call needs on the device: to count, depth and confidence; to
+    // write, the maps of what it writes.  One device block: the maps, the views, counts, offsets.
+    const bool write = positions != nullptr;
     auto a256 = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    for (int i = 0; i < n; ++i) {
-        const size_t px = (size_t)views[i].width * views[i].height;
-        off[i] = total;
-        total += a256(px * 4) + (views[i].normal ? a256(px * 12) : 0) +
-                 (views[i].confidence ? a256(px * 4) : 0) +
-                 (views[i].color ? a256(px * views[i].color_channels) : 0);
-        max_blocks = std::max(max_blocks, (px + kFuseBlock - 1) / kFuseBlock);
-    }
-    const size_t scan_off = total;
-    total += a256(max_blocks * 4) + a256(max_blocks * 8) + 256;
-    void* block = nullptr;
-    int rc = ctx->dev_alloc(&block, total, "fusion maps");
-    if (rc) return rc;
-    char* base = static_cast<char*>(block);
-    int* d_counts = reinterpret_cast<int*>(base + scan_off);
-    long long* d_offsets = reinterpret_cast<long long*>(base + scan_off + a256(max_blocks * 4));
-    long long* d_total = reinterpret_cast<long long*>(base + scan_off + a256(max_blocks * 4) +
-                                                      a256(max_blocks * 8));
     std::vector<FuseViewDev> g(n);
-    std::vector<HostLink::Seg> segs;
+    std::vector<HostLink::Seg> segs;   // device: offsets into the block, for now
+    size_t total = 0, blocks = 0;
+    auto put = [&](const void* host, size_t bytes) {
+        const size_t off = total;
+        segs.push_back({const_cast<void*>(host), reinterpret_cast<void*>(off), bytes});
+        total += a256(bytes);
+        return off;
+    };
+    struct Offsets { size_t depth, normal, conf, color; };
+    std::vector<Offsets> off(n);
     for (int i = 0; i < n; ++i) {
         const hp3d_fuse_view& v = views[i];
         const size_t px = (size_t)v.width * v.height;
-        char* p = base + off[i];
         FuseViewDev& d = g[i];
         std::memset(&d, 0, sizeof d);
         double ki[9];
-        if (hp3d_pm_invert3(v.K, ki) != HP3D_OK) {
-            ctx->dev_free(block, total);
+        if (hp3d_pm_invert3(v.K, ki) != HP3D_OK)
             return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: view %d K is singular", i);
-        }
         for (int k = 0; k < 9; ++k) { d.kinv[k] = (float)ki[k]; d.R[k] = (float)v.R[k]; }
         for (int k = 0; k < 3; ++k) d.t[k] = (float)v.t[k];
         d.W = v.width;
         d.H = v.height;
         d.channels = v.color ? v.color_channels : 0;
         d.min_conf = min_confidence;
-        d.depth = reinterpret_cast<float*>(p);
-        segs.push_back({const_cast<float*>(v.depth), p, px * 4});
-        p += a256(px * 4);
-        if (v.normal) {
-            d.normal = reinterpret_cast<float*>(p);
-            segs.push_back({const_cast<float*>(v.normal), p, px * 12});
-            p += a256(px * 12);
-        }
-        if (v.confidence) {
-            d.conf = reinterpret_cast<float*>(p);
-            segs.push_back({const_cast<float*>(v.confidence), p, px * 4});
-            p += a256(px * 4);
-        }
-        if (v.color) {
-            d.color = reinterpret_cast<uint8_t*>(p);
-            segs.push_back({const_cast<uint8_t*>(v.color), p, px * v.color_channels});
-        }
+        d.first_block = (int)blocks;
+        off[i].depth = put(v.depth, px * 4);
+        if (v.confidence) off[i].conf = put(v.confidence, px * 4);
+        if (write && normals && v.normal) off[i].normal = put(v.normal, px * 12);
+        if (write && colors && v.color) off[i].color = put(v.color, px * v.color_channels);
+        blocks += (px + kFuseSpan - 1) / kFuseSpan;
+    }
+    if (blocks > 0x7fffffff)
+        return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: %zu blocks of pixels", blocks);
+    const size_t views_off = put(g.data(), n * sizeof(FuseViewDev));
+    const size_t counts_off = total;
+    total += a256(blocks * 4) + a256(blocks * 8) + 256;
+    void* block = nullptr;
+    int rc = ctx->dev_alloc(&block, total, "fusion maps");
+    if (rc) return rc;
+    char* base = static_cast<char*>(block);
+    const FuseViewDev* d_views = reinterpret_cast<const FuseViewDev*>(base + views_off);
+    int* d_counts = reinterpret_cast<int*>(base + counts_off);
+    long long* d_offsets = reinterpret_cast<long long*>(base + counts_off + a256(blocks * 4));
+    long long* d_total = reinterpret_cast<long long*>(base + counts_off + a256(blocks * 4) +
+                                                      a256(blocks * 8));
+    for (auto& s : segs) s.dev = base + reinterpret_cast<size_t>(s.dev);
+    for (int i = 0; i < n; ++i) {
+        const hp3d_fuse_view& v = views[i];
+        g[i].depth = reinterpret_cast<const float*>(base + off[i].depth);
+        if (v.confidence) g[i].conf = reinterpret_cast<const float*>(base + off[i].conf);
+        if (write && normals && v.normal) g[i].normal = reinterpret_cast<const float*>(base + off[i].normal);
+        if (write && colors && v.color) g[i].color = reinterpret_cast<const uint8_t*>(base + off[i].color);
     }
     hipError_t e = ctx->link.upload(segs, ctx->stream);
-    // pass 1: count every view, in order, to size the output
-    std::vector<long long> view_base(n + 1, 0);
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
-        const int nb = (int)(((size_t)g[i].W * g[i].H + kFuseBlock - 1) / kFuseBlock);
-        hipLaunchKernelGGL(fuse_count_kernel, dim3(nb), dim3(kFuseBlock), 0, ctx->stream, g[i],
-                           d_counts);
-        hipLaunchKernelGGL(fuse_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_counts, nb,
-                           0ll, d_offsets, d_total);
-        long long t = 0;
+    long long npts_l = 0;
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(fuse_count_kernel, dim3((unsigned)blocks), dim3(kFuseBlock), 0,
+                           ctx->stream, d_views, n, d_counts);
+        hipLaunchKernelGGL(fuse_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_counts,
+                           (int)blocks, d_offsets, d_total);
         e = hipGetLastError();
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(&t, d_total, sizeof t, hipMemcpyDeviceToHost, ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        view_base[i + 1] = view_base[i] + t;
     }
+    if (e == hipSuccess) e = ctx->link.download({{&npts_l, d_total, sizeof npts_l}}, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
         ctx->dev_free(block, total);
         return ctx->hip_fail(e, "fusion count");
     }
-    const size_t npts = (size_t)view_base[n];
+    const size_t npts = (size_t)npts_l;
     *count = npts;
     if (!positions || npts == 0) {
         ctx->dev_free(block, total);
@@ -261,7 +297,7 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
         return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: %zu points exceed the capacity %zu", npts,
                          capacity);
     }
-    // pass 2: write into one device output block, then copy out
+    // write into one device output block, then copy out
     void* out = nullptr;
     const size_t per = npts * 12;
     const int nbuf = 1 + (normals ? 1 : 0) + (colors ? 1 : 0);
@@ -273,16 +309,9 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
     float* d_pos = static_cast<float*>(out);
     float* d_nrm = normals ? d_pos + 3 * npts : nullptr;
     float* d_col = colors ? d_pos + 3 * npts * (normals ? 2 : 1) : nullptr;
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
-        const int nb = (int)(((size_t)g[i].W * g[i].H + kFuseBlock - 1) / kFuseBlock);
-        hipLaunchKernelGGL(fuse_count_kernel, dim3(nb), dim3(kFuseBlock), 0, ctx->stream, g[i],
-                           d_counts);
-        hipLaunchKernelGGL(fuse_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_counts, nb,
-                           view_base[i], d_offsets, d_total);
-        hipLaunchKernelGGL(fuse_write_kernel, dim3(nb), dim3(kFuseBlock), 0, ctx->stream, g[i],
-                           d_offsets, d_pos, d_nrm, d_col);
-        e = hipGetLastError();
-    }
+    hipLaunchKernelGGL(fuse_write_kernel, dim3((unsigned)blocks), dim3(kFuseBlock), 0, ctx->stream,
+                       d_views, n, d_offsets, d_pos, d_nrm, d_col);
+    e = hipGetLastError();
     segs.assign({{positions, d_pos, per}});
     if (normals) segs.push_back({normals, d_nrm, per});
     if (colors) segs.push_back({colors, d_col, per});
