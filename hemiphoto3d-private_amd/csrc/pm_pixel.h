@@ -411,7 +411,9 @@ __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
                 sss = fmaf(sval, sval, sss);
                 srs = fmaf(r, sval, srs);
             }
-            __builtin_amdgcn_sched_barrier(0);   // no row's loads before the last row's samples
+            // (left to itself the compiler moves a chunk's loads among the last
+            // one's samples, until each is waited for by itself)
+            if (C < NT) __builtin_amdgcn_sched_barrier(0);
         }
     }
     m.sr = MASKED ? sr : wr.sr;
@@ -590,6 +592,11 @@ __device__ __forceinline__ float source_cost(const DevView& v, int s,
     // loop, which gives the same result).
     const bool inside = window_inside(cx, cy, cz, h00, h01, h10, h11, h20, h21, (float)R,
                                       Wq, Hq);
+    // Where the masked loop has a third form without the per-tap |w_z| test: it
+    // gains 2 % with FP16 storage and 1-3 % with FP32 at stride 1 (1280x960, 8
+    // sources, 11 x 11 taps: 1.84 -> 1.81 ms a half-pass; 800x600, 5 x 5: 86.8 ->
+    // 84.8 us), and loses 2 % with FP32 at stride 2 and 3 % in the 11-tap FP32 cost.
+    constexpr bool kZClear = STORE == kStoreF16 || (ST == 1 && (NT <= 7 || C < NT));
     TapSums m;
     // No tap of any lane's window in the image: the cost is that of no sample.
     // (9 % of the wave evaluations of a 4-source 30-degree arc, image-edge
@@ -605,9 +612,7 @@ __device__ __forceinline__ float source_cost(const DevView& v, int s,
     if (__all(inside)) {
         tap_window<NT, ST, STORE, false, true, C>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
                                                    t11, h20, h21, umax, vmax, wr, m, bu, bv);
-    } else if (STORE == kStoreF16 && __all(z_clear(cz, h20, h21, (float)R))) {
-        // FP16 storage only: a third loop without the per-tap |w_z| test
-        // measured +2 % there and -12 % with FP32 storage at stride 1
+    } else if (kZClear && __all(z_clear(cz, h20, h21, (float)R))) {
         tap_window<NT, ST, STORE, true, false, C>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
                                                    t11, h20, h21, umax, vmax, wr, m, bu, bv);
     } else {

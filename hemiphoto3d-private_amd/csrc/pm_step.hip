@@ -9,8 +9,8 @@
 // views can join between steps.
 //
 // Work decomposition: every view is cut into TX x TY compacted tiles; all
-// items' tiles form one logical range, cut into chunks of kStepChunk
-// consecutive tiles.  Workgroups are dispatched to the 8 XCDs round-robin
+// items' tiles form one logical range, cut into chunks of consecutive
+// tiles.  Workgroups are dispatched to the 8 XCDs round-robin
 // (block b -> XCD b % 8); XCD x takes chunks x, x + 8, x + 16, ... in order.
 // Tiles of a chunk are neighbours in one view and read the same source rows
 // through that XCD's L2, while every XCD sees an even sample of the whole
@@ -28,7 +28,17 @@
 
 namespace hp3d {
 
-constexpr int kStepChunk = 16;   // tiles per chunk of the XCD interleave
+// Chunks of the XCD interleave, as powers of two.  A chunk's neighbours share
+// rows of the sources in that XCD's L2, and FP32's planes need twice as much of
+// it: four views of 640x480 to 2400x1800, 6 x 6 taps, FP32, 35.3 ms in chunks of
+// 16, 34.7 of 64; one 1600x1200 view, 11 x 11 taps, FP32, 22.8 against 22.1;
+// FP16 16.5 in chunks of 16, 16.3 of 32 or 64.  A step of few tiles keeps
+// smaller ones, so that every XCD has at least kStepChunksPerXcd (with 4 or 16
+// of them instead of 8: 22.4 and 22.5 ms for that one view), but not below 16:
+// two 320x240 views in chunks of 4, 1.08 against 1.07 ms.
+constexpr int kStepChunkMin = 4;
+template <int STORE> constexpr int kStepChunkMax = STORE == kStoreF32 ? 6 : 5;
+constexpr int kStepChunksPerXcd = 8;
 constexpr int kPersistMaxGrid = 4096;
 // Waves per SIMD that every step kernel's registers must allow (128): only the
 // 11-tap FP32 instances need asking (134 registers without), and do not spill.
@@ -37,16 +47,17 @@ constexpr int kStepWaves = 4;
 template <int NT, int ST, int STORE, int TX, int TY, int WPE>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE < kStepWaves ? kStepWaves : WPE, 8)))
 void pm_step_kernel(const DevJob* __restrict__ jobs, const StepItem* __restrict__ items,
-                    int n_items, int total_tiles)
+                    int n_items, int total_tiles, int chunk_log2)
 {
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
     __shared__ float tile[G::LH * G::LP];
     __shared__ PassXchg<TX * TY> xc;
 
-    const int b = blockIdx.x;                       // gridDim.x: a multiple of 8 * kStepChunk
+    const int b = blockIdx.x;                       // gridDim.x: a multiple of 8 chunks
     const int sidx = b >> 3;                        // position in this XCD's sequence
-    const int t = ((sidx / kStepChunk) * 8 + (b & 7)) * kStepChunk + sidx % kStepChunk;
+    const int t = ((((sidx >> chunk_log2) << 3) + (b & 7)) << chunk_log2) +
+                  (sidx & ((1 << chunk_log2) - 1));
     if (t >= total_tiles) return;
     int lo = 0, hi = n_items - 1;                   // last item with tile_begin <= t
     while (lo < hi) {
@@ -343,10 +354,13 @@ template <int NT, int ST, int STORE, int TX, int TY, int WPE>
 static hipError_t launch_t(const DevJob* jobs, const StepItem* items, int n_items, int total_tiles,
                            hipStream_t st)
 {
-    constexpr int kGroup = 8 * kStepChunk;
-    const int grid = ((total_tiles + kGroup - 1) / kGroup) * kGroup;
+    int chunk_log2 = kStepChunkMax<STORE>;
+    while (chunk_log2 > kStepChunkMin && (total_tiles >> chunk_log2) < 8 * kStepChunksPerXcd)
+        --chunk_log2;
+    const int group = 8 << chunk_log2;
+    const int grid = ((total_tiles + group - 1) / group) * group;
     hipLaunchKernelGGL((pm_step_kernel<NT, ST, STORE, TX, TY, WPE>), dim3(grid), dim3(TX * TY), 0,
-                       st, jobs, items, n_items, total_tiles);
+                       st, jobs, items, n_items, total_tiles, chunk_log2);
     return hipGetLastError();
 }
 
