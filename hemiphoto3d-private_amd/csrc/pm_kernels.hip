@@ -64,7 +64,16 @@ __global__ __launch_bounds__(TX * TY) void pm_cost_kernel(DevView v, int tiles_x
 #define HP3D_PLAIN_WPE 4
 #endif
 
-template <int NT, int ST, int STORE, int TX, int TY>
+// The pooled form of the refinement pays from 6 taps a row (1600x1200, 4 sources,
+// FP32: 415 -> 402 us a half-pass; with 5 x 5 taps, 800x600, 3 sources, 80.7 ->
+// 78.3 in means over three, but a whole solve 989 -> 1000 us over two; 3 x 3 taps,
+// 1600x1200, 2 sources, 110 -> 112) and from about 3 workgroups to a CU on, where
+// others fill the waits at its barriers (tiles of 32 x 8: 720x540, 816 tiles, 259
+// -> 248 us with 3 sources and 11 x 11 taps; 640x480, 600 tiles, 77.2 -> 78.7 with
+// 2 and 7 x 7; 480x360, 345 tiles, 66 -> 69 with 3 and 6 x 6).
+constexpr int kPoolTaps = 6, kPoolTiles = 768;
+
+template <int NT, int ST, int STORE, int TX, int TY, bool POOL>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(HP3D_PLAIN_WPE, 8)))
 void pm_halfpass_kernel(DevView v, int iteration, int parity, uint64_t pass_seed, int tiles_x,
                         int tiles)
@@ -77,7 +86,7 @@ void pm_halfpass_kernel(DevView v, int iteration, int parity, uint64_t pass_seed
     if (!xcd_tile(tiles_x, tiles, bx, by)) return;
     stage_ref_tile<R, STORE, TX, TY>(v, tile, bx, by);
     halfpass_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, threadIdx.x % TX, threadIdx.x / TX,
-                                          iteration, parity, pass_seed, xc);
+                                          iteration, parity, pass_seed, xc, POOL);
 }
 
 // Views of few pixels: up to kMaxSplitWaves waves for 64 pixels (halfpass_split).
@@ -322,9 +331,14 @@ static void launch_pass_t(const DevView& v, int mode, int iteration, int parity,
     if (mode == kPassCost)
         hipLaunchKernelGGL((pm_cost_kernel<NT, ST, STORE, kTX, kTY>), dim3(xcd_grid(2 * tiles)),
                            dim3(kTX * kTY), kIdleLds, st, v, tiles_x, tiles);
+    else if (NT >= kPoolTaps && tiles >= kPoolTiles && pool_refinement(v.S, v.top_k, iteration))
+        hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY, (NT >= kPoolTaps)>),
+                           dim3(xcd_grid(tiles)), dim3(kTX * kTY), 0, st, v, iteration, parity,
+                           pass_seed, tiles_x, tiles);
     else
-        hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY>), dim3(xcd_grid(tiles)),
-                           dim3(kTX * kTY), 0, st, v, iteration, parity, pass_seed, tiles_x, tiles);
+        hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY, false>),
+                           dim3(xcd_grid(tiles)), dim3(kTX * kTY), 0, st, v, iteration, parity,
+                           pass_seed, tiles_x, tiles);
 }
 
 template <int STORE>

@@ -663,6 +663,18 @@ struct TopCosts {
         }
         top[0] = fminf(c, top[0]);
     }
+    // What mean() cannot be below once one more cost (>= 0) is inserted: the same
+    // sum, of entries none of which is larger, and rounding keeps that order.
+    // Only for means of two or three.
+    __device__ __forceinline__ float bound(const DevView& v) const
+    {
+        const int k = v.top_k < v.S ? v.top_k : v.S;
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (i < k - 1) sum += top[i];
+        return sum / (float)k;
+    }
     __device__ __forceinline__ float mean(const DevView& v) const
     {
         const int k = v.top_k < v.S ? v.top_k : v.S;
@@ -784,7 +796,19 @@ template <int T> struct PassXchg {
     WinRef wref[T];
     int hist[T];        // 64 depth buckets per wave
     int wsum[T / 64];   // entries per wave
+    int rsum[2][T / 64];   // refinement candidates per wave that need their last source
 };
+
+// Where halfpass_pixel pools the refinement candidates' last source (at its
+// loop): a bound needs a mean over two or three of at least two sources, and from
+// the seventh iteration on the candidates lie so near the current hypothesis that
+// few are rejected before it (640x480, 4 sources, 6 x 6 taps, the first step's
+// candidates: 59, 74, 67 and 41 % in the first, second, fourth and sixth
+// iteration, 12 % in the eighth).
+__host__ __device__ __forceinline__ bool pool_refinement(int S, int top_k, int iteration)
+{
+    return S >= 2 && top_k >= 2 && top_k <= 3 && iteration < 6;
+}
 
 // Depth buckets of a wave's counting sort: inverse depth (disparity) over the
 // view's range.
@@ -908,11 +932,13 @@ __device__ __forceinline__ float4 refine_cand(const float4& best, const uint4& w
 // pixel's candidate (all windows of the workgroup are in LDS), and each
 // owner then applies the costs in L, R, U, D order.  The result is the one
 // the plain per-lane loop gives, with fewer evaluation rounds.
-// Every thread of the workgroup must call this (it synchronises the group).
+// Every thread of the workgroup must call this (it synchronises the group),
+// with the same pool (see pool_refinement).
 template <int NT, int ST, int STORE, int TX, int TY, bool COH = false>
 __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* tile, int bx, int by,
                                                int tx, int ty, int iteration, int parity,
-                                               uint64_t pass_seed, PassXchg<TX * TY>& xc)
+                                               uint64_t pass_seed, PassXchg<TX * TY>& xc,
+                                               bool pool = false)
 {
     constexpr int R = (NT - 1) * ST / 2, T = TX * TY;
     using G = TileGeom<R, STORE, TX, TY>;
@@ -1067,7 +1093,7 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
         }
     }
     __syncthreads();
-    if (!active) return;
+    if (!pool && !active) return;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (!((need >> k) & 1u)) continue;
@@ -1075,25 +1101,113 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
         if (c < bc) { bc = c; best = xc.hyp[t + k * T]; changed = true; }
     }
 
-    double rx, ry, rz;
-    ray_fp64(v.kinv_d, x, y, rx, ry, rz);
-    float ux, uy, uz;
-    unit_ray(v.kinv, x, y, ux, uy, uz);
     float depth_range = (dmax - dmin) * 0.5f;
     float normal_range = 1.0f;
     for (int it = 0; it < iteration; ++it) { depth_range *= 0.6f; normal_range *= 0.6f; }
     const uint32_t idx = (uint32_t)(y * v.W + x);
+    if (pool) {
+        // A candidate whose mean without its last source cannot be below the
+        // current cost is not accepted whatever that source says.  After the
+        // other sources the workgroup lists the lanes that still need it, and
+        // where they fit into fewer rounds than it has waves, wave w evaluates the
+        // last source of entries 64 w .. 64 w + 63.  Rejected or not, the costs
+        // that are compared are those of the plain loop below.  (Half-passes of
+        // 8-iteration solves: 2400x1800, 4 sources, 6 x 6 taps, FP16 879 -> 838 us;
+        // 1280x960, 8 sources, 11 x 11, FP32 1610 -> 1567; 3 sources, 7 x 7 286 ->
+        // 276.  The neighbours' list the same way gained nothing: fewer of them are
+        // rejected, and every group of T entries waits for its slowest wave.)
 #pragma unroll 1
-    for (int step = 0; step < 2; ++step) {
-        uint32_t c0 = idx, c1 = (uint32_t)iteration, c2 = (uint32_t)step, c3 = kDomainRefine;
-        philox(c0, c1, c2, c3, (uint32_t)pass_seed, (uint32_t)(pass_seed >> 32));
-        const float4 cand = refine_cand(best, make_uint4(c0, c1, c2, c3), depth_range,
-                                        normal_range, dmin, dmax, ux, uy, uz);
-        const float c = cand_cost<NT, ST, STORE, kPassChunk<NT>>(v, lwin, G::LP, wr, x, y, rx, ry, rz, cand.x,
-                                                 cand.y, cand.z, cand.w);
-        if (c < bc) { bc = c; best = cand; changed = true; }
-        depth_range *= 0.5f;
-        normal_range *= 0.5f;
+        for (int step = 0; step < 2; ++step) {
+            float4 cand = make_float4(0.f, 0.f, 0.f, 0.f);
+            int xe = x, ye = y;
+            const float* lwe = lwin;
+            WinRef we = xc.wref[t];
+            CandPlane g;
+            bool live = active;
+            if (active) {
+                uint32_t c0 = idx, c1 = (uint32_t)iteration, c2 = (uint32_t)step, c3 = kDomainRefine;
+                philox(c0, c1, c2, c3, (uint32_t)pass_seed, (uint32_t)(pass_seed >> 32));
+                float ux, uy, uz;
+                unit_ray(v.kinv, x, y, ux, uy, uz);
+                cand = refine_cand(best, make_uint4(c0, c1, c2, c3), depth_range, normal_range,
+                                   dmin, dmax, ux, uy, uz);
+                xc.hyp[t] = cand;
+                double rx, ry, rz;
+                ray_fp64(v.kinv_d, x, y, rx, ry, rz);
+                live = cand_plane(v, x, y, rx, ry, rz, cand.x, cand.y, cand.z, cand.w, g);
+            }
+            bool run = live, pooled = false;
+            int place = 0;
+            TopCosts top;
+            for (int s = 0; s < v.S; ++s) {
+                if (s == v.S - 1) {
+                    live = live && top.bound(v) < bc;
+                    const unsigned long long m = __ballot(live);
+                    if (lane == 0) xc.rsum[step][t >> 6] = __popcll(m);
+                    __syncthreads();
+                    int all = 0;
+                    place = __popcll(m & below);
+#pragma unroll
+                    for (int w = 0; w < T / 64; ++w) {
+                        const int c = xc.rsum[step][w];
+                        if (w < (t >> 6)) place += c;
+                        all += c;
+                    }
+                    all = __builtin_amdgcn_readfirstlane(all);
+                    pooled = all <= T - 64;
+                    run = live;
+                    if (pooled) {
+                        if (live) xc.item[place] = (unsigned short)t;
+                        __syncthreads();
+                        run = t < all;
+                        if (run) {
+                            const int t_o = xc.item[t];
+                            const int tx_o = t_o % TX, ty_o = t_o / TX;
+                            ye = by * TY + ty_o;
+                            xe = 2 * (bx * TX + tx_o) + ((ye + parity) & 1);
+                            lwe = tile + ty_o * G::LP + (xe - 2 * bx * TX);
+                            we = xc.wref[t_o];
+                            const float4 h = xc.hyp[t_o];
+                            double qx, qy, qz;
+                            ray_fp64(v.kinv_d, xe, ye, qx, qy, qz);
+                            cand_plane(v, xe, ye, qx, qy, qz, h.x, h.y, h.z, h.w, g);
+                        }
+                    }
+                }
+                if (run) {
+                    const float c = source_cost<NT, ST, STORE, kPassChunk<NT>>(v, s, lwe, G::LP, we,
+                                                                               xe, ye, g);
+                    if (pooled) xc.cost[t] = c;
+                    else top.insert(c, true);
+                }
+            }
+            if (pooled) {
+                __syncthreads();
+                if (live) top.insert(xc.cost[place], true);
+            }
+            const float c = top.mean(v);
+            if (live && c < bc) { bc = c; best = cand; changed = true; }
+            depth_range *= 0.5f;
+            normal_range *= 0.5f;
+        }
+        if (!active) return;
+    } else {
+        double rx, ry, rz;
+        ray_fp64(v.kinv_d, x, y, rx, ry, rz);
+        float ux, uy, uz;
+        unit_ray(v.kinv, x, y, ux, uy, uz);
+#pragma unroll 1
+        for (int step = 0; step < 2; ++step) {
+            uint32_t c0 = idx, c1 = (uint32_t)iteration, c2 = (uint32_t)step, c3 = kDomainRefine;
+            philox(c0, c1, c2, c3, (uint32_t)pass_seed, (uint32_t)(pass_seed >> 32));
+            const float4 cand = refine_cand(best, make_uint4(c0, c1, c2, c3), depth_range,
+                                            normal_range, dmin, dmax, ux, uy, uz);
+            const float c = cand_cost<NT, ST, STORE, kPassChunk<NT>>(v, lwin, G::LP, wr, x, y, rx, ry, rz, cand.x,
+                                                     cand.y, cand.z, cand.w);
+            if (c < bc) { bc = c; best = cand; changed = true; }
+            depth_range *= 0.5f;
+            normal_range *= 0.5f;
+        }
     }
     IO::st4(own, p, best);
     IO::st1(v.cost[parity], p, bc);

@@ -39,6 +39,12 @@ namespace hp3d {
 constexpr int kStepChunkMin = 4;
 template <int STORE> constexpr int kStepChunkMax = STORE == kStoreF32 ? 6 : 5;
 constexpr int kStepChunksPerXcd = 8;
+// Steps with the refinement's pooled form: windows of 7 x 7 taps and more, and
+// tiles to fill the chip (one 1600x1200 view, 11 x 11 taps, FP32: 22.1 -> 20.9 ms;
+// a mixed FP16 batch 106.6 -> 102.9; with 6 x 6 taps FP16 16.35 -> 16.26, FP32
+// 34.7 -> 34.6 and small batches 2-4 % slower, its instances being at their limit
+// of registers).
+constexpr int kPoolStepTaps = 7, kPoolStepTiles = 1024;
 constexpr int kPersistMaxGrid = 4096;
 // Waves per SIMD that every step kernel's registers must allow (128): only the
 // 11-tap FP32 instances need asking (134 registers without), and do not spill.
@@ -47,7 +53,7 @@ constexpr int kStepWaves = 4;
 template <int NT, int ST, int STORE, int TX, int TY, int WPE>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE < kStepWaves ? kStepWaves : WPE, 8)))
 void pm_step_kernel(const DevJob* __restrict__ jobs, const StepItem* __restrict__ items,
-                    int n_items, int total_tiles, int chunk_log2)
+                    int n_items, int total_tiles, int chunk_log2, int pool)
 {
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
@@ -85,7 +91,9 @@ void pm_step_kernel(const DevJob* __restrict__ jobs, const StepItem* __restrict_
         cost_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, tx, ty, 1);
     } else {
         halfpass_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, tx, ty, it.iteration, it.parity,
-                                              it.pass_seed, xc);
+                                              it.pass_seed, xc,
+                                              NT >= kPoolStepTaps && pool &&
+                                                  pool_refinement(v.S, v.top_k, it.iteration));
     }
     // outputs: this lane's pixel of each colour; the other colour was
     // completed by the previous step
@@ -360,7 +368,8 @@ static hipError_t launch_t(const DevJob* jobs, const StepItem* items, int n_item
     const int group = 8 << chunk_log2;
     const int grid = ((total_tiles + group - 1) / group) * group;
     hipLaunchKernelGGL((pm_step_kernel<NT, ST, STORE, TX, TY, WPE>), dim3(grid), dim3(TX * TY), 0,
-                       st, jobs, items, n_items, total_tiles, chunk_log2);
+                       st, jobs, items, n_items, total_tiles, chunk_log2,
+                       total_tiles >= kPoolStepTiles ? 1 : 0);
     return hipGetLastError();
 }
 
