@@ -16,7 +16,7 @@
 //     warp, one v_rcp_f32, one buffer load (the quad from the
 //     row-difference plane) and 4 instructions for the bilinear sample;
 //   * neighbour candidates that provably cannot win are skipped and the rest
-//     shared across the wave's lanes (halfpass_pixel in pm_pixel.h);
+//     shared over the workgroup's lanes (halfpass_pixel in pm_pixel.h);
 //   * the five NCC moments are accumulated in FP32 on values shifted by
 //     -128 DN; the variance cancellation is done in FP64.
 #include <hip/hip_runtime.h>
