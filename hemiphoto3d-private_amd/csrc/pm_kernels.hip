@@ -57,9 +57,9 @@ __global__ __launch_bounds__(TX * TY) void pm_cost_kernel(DevView v, int tiles_x
 }
 
 // Minimum waves per SIMD the half-pass's register allocation must allow.  4:
-// every window's kernel fits 128 registers (7 x 7 taps with FP32 planes, 129
-// unasked, keeps three SGPRs' worth of spills outside its loops), and a pass
-// issues a vector instruction nearly every 4 clocks; 5 would spill in the loops.
+// every window's kernel fits 128 registers without spilling one (up to 40 scalar
+// registers go to lanes of vector ones), and a pass issues a vector instruction
+// nearly every 4 clocks; 5 would spill in the loops.
 #ifndef HP3D_PLAIN_WPE
 #define HP3D_PLAIN_WPE 4
 #endif

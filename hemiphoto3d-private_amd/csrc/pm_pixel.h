@@ -1118,10 +1118,10 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
         // rejected, and every group of T entries waits for its slowest wave.)
 #pragma unroll 1
         for (int step = 0; step < 2; ++step) {
-            float4 cand = make_float4(0.f, 0.f, 0.f, 0.f);
-            int xe = x, ye = y;
-            const float* lwe = lwin;
-            WinRef we = xc.wref[t];
+            // (what can be read from LDS or formed again is: held in registers
+            // through the sources, the candidate, its pixel and its window sums took
+            // the 6-tap and 7-tap FP32 kernels past 128, with two spilled to scratch)
+            int te = t;   // the owner of the candidate that this lane evaluates
             CandPlane g;
             bool live = active;
             if (active) {
@@ -1129,8 +1129,8 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
                 philox(c0, c1, c2, c3, (uint32_t)pass_seed, (uint32_t)(pass_seed >> 32));
                 float ux, uy, uz;
                 unit_ray(v.kinv, x, y, ux, uy, uz);
-                cand = refine_cand(best, make_uint4(c0, c1, c2, c3), depth_range, normal_range,
-                                   dmin, dmax, ux, uy, uz);
+                const float4 cand = refine_cand(best, make_uint4(c0, c1, c2, c3), depth_range,
+                                                normal_range, dmin, dmax, ux, uy, uz);
                 xc.hyp[t] = cand;
                 double rx, ry, rz;
                 ray_fp64(v.kinv_d, x, y, rx, ry, rz);
@@ -1161,13 +1161,10 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
                         __syncthreads();
                         run = t < all;
                         if (run) {
-                            const int t_o = xc.item[t];
-                            const int tx_o = t_o % TX, ty_o = t_o / TX;
-                            ye = by * TY + ty_o;
-                            xe = 2 * (bx * TX + tx_o) + ((ye + parity) & 1);
-                            lwe = tile + ty_o * G::LP + (xe - 2 * bx * TX);
-                            we = xc.wref[t_o];
-                            const float4 h = xc.hyp[t_o];
+                            te = xc.item[t];
+                            const int ye = by * TY + te / TX;
+                            const int xe = 2 * (bx * TX + te % TX) + ((ye + parity) & 1);
+                            const float4 h = xc.hyp[te];
                             double qx, qy, qz;
                             ray_fp64(v.kinv_d, xe, ye, qx, qy, qz);
                             cand_plane(v, xe, ye, qx, qy, qz, h.x, h.y, h.z, h.w, g);
@@ -1175,8 +1172,11 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
                     }
                 }
                 if (run) {
-                    const float c = source_cost<NT, ST, STORE, kPassChunk<NT>>(v, s, lwe, G::LP, we,
-                                                                               xe, ye, g);
+                    const int ye = by * TY + te / TX;
+                    const int xe = 2 * (bx * TX + te % TX) + ((ye + parity) & 1);
+                    const float c = source_cost<NT, ST, STORE, kPassChunk<NT>>(
+                        v, s, tile + te / TX * G::LP + (xe - 2 * bx * TX), G::LP, xc.wref[te], xe,
+                        ye, g);
                     if (pooled) xc.cost[t] = c;
                     else top.insert(c, true);
                 }
@@ -1186,7 +1186,7 @@ __device__ __forceinline__ void halfpass_pixel(const DevView& v, const float* ti
                 if (live) top.insert(xc.cost[place], true);
             }
             const float c = top.mean(v);
-            if (live && c < bc) { bc = c; best = cand; changed = true; }
+            if (live && c < bc) { bc = c; best = xc.hyp[t]; changed = true; }
             depth_range *= 0.5f;
             normal_range *= 0.5f;
         }
