@@ -249,8 +249,10 @@ hipError_t launch_plan(hp3d_pm_ctx* ctx, const Plan& p, int store, int radius, i
     const StepItem* items = static_cast<const StepItem*>(ctx->batch_items.ptr);
     for (size_t s = 0; s < p.count.size(); ++s) {
         if (p.count[s] == 0) continue;
+        // (the views of a plan's step are all at the same step)
+        const bool start = p.items[p.offset[s]].mode == kStepStart;
         hipError_t e = launch_step(store, radius, stride, variant, jobs, items + p.offset[s],
-                                   p.count[s], p.tiles[s], ctx->stream);
+                                   p.count[s], p.tiles[s], start, ctx->stream);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

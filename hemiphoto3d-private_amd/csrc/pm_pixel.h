@@ -752,7 +752,7 @@ __device__ __forceinline__ float4 init_hyp(const DevView& v, int x, int y, uint6
 
 // Cost of the current hypothesis of the colour-`parity` pixel of lane (tx, ty)
 // in tile (bx, by); returns false if the lane has no pixel.
-template <int NT, int ST, int STORE, int TX, int TY, bool COH = false>
+template <int NT, int ST, int STORE, int TX, int TY, int C = kCostChunk<NT>, bool COH = false>
 __device__ __forceinline__ bool cost_pixel(const DevView& v, const float* tile, int bx, int by,
                                            int tx, int ty, int parity)
 {
@@ -769,7 +769,7 @@ __device__ __forceinline__ bool cost_pixel(const DevView& v, const float* tile, 
     const float4 h = StateIO<COH>::ld4(v.hyp[parity], p);
     const WinRef wr = window_ref_sums<NT, ST>(lwin, G::LP);
     StateIO<COH>::st1(v.cost[parity], p,
-                      cand_cost<NT, ST, STORE, kCostChunk<NT>>(v, lwin, G::LP, wr, x, y, rx, ry, rz, h.x, h.y,
+                      cand_cost<NT, ST, STORE, C>(v, lwin, G::LP, wr, x, y, rx, ry, rz, h.x, h.y,
                                                   h.z, h.w));
     return true;
 }

@@ -427,7 +427,7 @@ void hp3d_pm_server::loop()
             if (e == hipSuccess) e = hipEventRecord(ev_a[b], compute);
             if (e == hipSuccess)
                 e = launch_step(o.store, o.radius, o.stride, variant, d_jobs, d_items[b], n_items,
-                                total_tiles, compute);
+                                total_tiles, (int)fresh.size() == n_items, compute);
             if (e == hipSuccess) e = hipEventRecord(ev_b[b], compute);
             // jobs whose last step this was go to the completion thread only
             // once the event it waits on is recorded

@@ -41,7 +41,7 @@ enum PersistCtl : int { kCtlQueue0 = 0, kCtlAbort = 8, kCtlWords = 9 };
 
 struct StepVariant {
     int tx, ty;        // compacted columns x rows per workgroup
-    int wpe;           // minimum waves per SIMD requested from the compiler
+    int wpe;           // minimum waves per SIMD that the variant asks the compiler for
 };
 extern const StepVariant kStepVariants[];
 extern const int kNumStepVariants;
@@ -56,8 +56,10 @@ constexpr int kDefaultStepVariant = 1;
 int step_tile_tx(int variant);
 int step_tile_ty(int variant);
 
+// start_only: every item is a START.
 hipError_t launch_step(int store, int radius, int stride, int variant, const DevJob* jobs,
-                       const StepItem* items, int n_items, int total_tiles, hipStream_t st);
+                       const StepItem* items, int n_items, int total_tiles, bool start_only,
+                       hipStream_t st);
 
 // One launch for a whole batch: items of every step in step order, their
 // tile_begin counting units (tiles) across all steps; done holds one counter

@@ -46,14 +46,39 @@ constexpr int kStepChunksPerXcd = 8;
 // of registers).
 constexpr int kPoolStepTaps = 7, kPoolStepTiles = 1024;
 constexpr int kPersistMaxGrid = 4096;
-// Waves per SIMD that every step kernel's registers must allow (128): only the
-// 11-tap FP32 instances need asking (134 registers without), and do not spill.
-constexpr int kStepWaves = 4;
+// What a step's items are, a kernel instance each.
+enum StepForm : int { kFormPlain, kFormPooled, kFormStart };   // kFormStart: START items only
 
-template <int NT, int ST, int STORE, int TX, int TY, int WPE>
-__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(WPE < kStepWaves ? kStepWaves : WPE, 8)))
+// Waves per SIMD that an instance's registers must allow.  Most fit 4 (128
+// registers) unasked, and asking all the same made the compiler order the START
+// items' gathers worse (one 1600x1200 view, FP32: START 0.711 -> 0.887 ms with
+// 9 x 9 taps, 0.347 -> 0.386 with 6 x 6).  Asked for where it is 3 otherwise:
+//   11 x 11 FP32 pooled (135 registers; at 128 it spills 8): such a view's solve
+//     21.7 ms with 3 waves, 21.0 with 4; its rows in chunks of 4, without spills,
+//     22.2;
+//   7 x 7 pooled (144 FP32, 138 FP16; 15 and 2 spilled) and 7 x 7 FP32 (132; none
+//     spilled): 801x601, 3 sources, FP32 2.72 ms with 3 waves, 2.21 with 4; in
+//     chunks of 4, without spills, 3 to 5 % slower.
+// No spilled register is reloaded in the tap loops of a half-pass.
+template <int NT, int ST, int STORE, int FORM>
+constexpr int kStepWaves =
+    ST == 1 && ((NT == 11 && STORE == kStoreF32 && FORM == kFormPooled) ||
+                (NT == 7 && (FORM == kFormPooled || (FORM == kFormPlain && STORE == kStoreF32))))
+        ? 4 : 1;
+// Whether a step of START items alone has an instance of its own: 7 x 7 windows,
+// whose START the 4 waves slow down (1600x1200, 4 sources, FP32: 0.448 ms unasked,
+// 0.531 asked for).
+template <int NT, int ST> constexpr bool kStartForm = NT == 7 && ST == 1;
+// Taps of a row in flight in a START item's cost: the initial cost's whole rows;
+// 11 FP32 quads in flight there would take the plain form to 137 registers, 3 waves
+// (START as fast either way: 2.05 against 2.04 ms for 640x480 to 1600x1200 views).
+template <int NT, int STORE>
+constexpr int kStartChunk = NT == 11 && STORE == kStoreF32 ? kPassChunk<NT> : kCostChunk<NT>;
+
+template <int NT, int ST, int STORE, int TX, int TY, int FORM>
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu((kStepWaves<NT, ST, STORE, FORM>), 8)))
 void pm_step_kernel(const DevJob* __restrict__ jobs, const StepItem* __restrict__ items,
-                    int n_items, int total_tiles, int chunk_log2, int pool)
+                    int n_items, int total_tiles, int chunk_log2)
 {
     constexpr int R = (NT - 1) * ST / 2;
     using G = TileGeom<R, STORE, TX, TY>;
@@ -80,19 +105,19 @@ void pm_step_kernel(const DevJob* __restrict__ jobs, const StepItem* __restrict_
 
     stage_ref_tile<R, STORE, TX, TY>(v, tile, bx, by);
     const int i = bx * TX + tx, y = by * TY + ty;
-    if (it.mode == kStepStart) {
+    if (FORM == kFormStart || it.mode == kStepStart) {
         if (y < v.H) {
             for (int c = 0; c < 2; ++c) {
                 const int x = 2 * i + ((y + c) & 1);
                 if (x < v.W) v.hyp[c][y * v.Wc + i] = init_hyp(v, x, y, job.seed);
             }
         }
-        cost_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, tx, ty, 0);
-        cost_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, tx, ty, 1);
+        cost_pixel<NT, ST, STORE, TX, TY, kStartChunk<NT, STORE>>(v, tile, bx, by, tx, ty, 0);
+        cost_pixel<NT, ST, STORE, TX, TY, kStartChunk<NT, STORE>>(v, tile, bx, by, tx, ty, 1);
     } else {
         halfpass_pixel<NT, ST, STORE, TX, TY>(v, tile, bx, by, tx, ty, it.iteration, it.parity,
                                               it.pass_seed, xc,
-                                              NT >= kPoolStepTaps && pool &&
+                                              FORM == kFormPooled &&
                                                   pool_refinement(v.S, v.top_k, it.iteration));
     }
     // outputs: this lane's pixel of each colour; the other colour was
@@ -250,8 +275,8 @@ void pm_persist_kernel(const DevJob* __restrict__ jobs, const StepItem* __restri
                         if (x < v.W) StateIO<true>::st4(v.hyp[c], y * v.Wc + i, init_hyp(v, x, y, job.seed));
                     }
                 }
-                cost_pixel<NT, ST, STORE, TX, TY, true>(v, tile, bx, by, tx, ty, 0);
-                cost_pixel<NT, ST, STORE, TX, TY, true>(v, tile, bx, by, tx, ty, 1);
+                cost_pixel<NT, ST, STORE, TX, TY, kCostChunk<NT>, true>(v, tile, bx, by, tx, ty, 0);
+                cost_pixel<NT, ST, STORE, TX, TY, kCostChunk<NT>, true>(v, tile, bx, by, tx, ty, 1);
             } else {
                 halfpass_pixel<NT, ST, STORE, TX, TY, true>(v, tile, bx, by, tx, ty, it.iteration,
                                                             it.parity, it.pass_seed,
@@ -358,24 +383,33 @@ hipError_t launch_persistent(int store, int radius, int stride, int variant, con
 // batched and serving workloads (radius 5, stride 1 or 2) also have the tile
 // shapes and occupancies the autotuner chooses from.
 // ---------------------------------------------------------------------------
-template <int NT, int ST, int STORE, int TX, int TY, int WPE>
+template <int NT, int ST, int STORE, int TX, int TY>
 static hipError_t launch_t(const DevJob* jobs, const StepItem* items, int n_items, int total_tiles,
-                           hipStream_t st)
+                           bool start_only, hipStream_t st)
 {
     int chunk_log2 = kStepChunkMax<STORE>;
     while (chunk_log2 > kStepChunkMin && (total_tiles >> chunk_log2) < 8 * kStepChunksPerXcd)
         --chunk_log2;
     const int group = 8 << chunk_log2;
-    const int grid = ((total_tiles + group - 1) / group) * group;
-    hipLaunchKernelGGL((pm_step_kernel<NT, ST, STORE, TX, TY, WPE>), dim3(grid), dim3(TX * TY), 0,
-                       st, jobs, items, n_items, total_tiles, chunk_log2,
-                       total_tiles >= kPoolStepTiles ? 1 : 0);
+    const dim3 grid(((total_tiles + group - 1) / group) * group), block(TX * TY);
+    // (a form that a window does not have is an instance of its plain one)
+    constexpr int kStart = kStartForm<NT, ST> ? kFormStart : kFormPlain;
+    constexpr int kPooled = NT >= kPoolStepTaps ? kFormPooled : kFormPlain;
+    if (start_only && kStartForm<NT, ST>)
+        hipLaunchKernelGGL((pm_step_kernel<NT, ST, STORE, TX, TY, kStart>), grid, block, 0, st, jobs,
+                           items, n_items, total_tiles, chunk_log2);
+    else if (!start_only && total_tiles >= kPoolStepTiles)
+        hipLaunchKernelGGL((pm_step_kernel<NT, ST, STORE, TX, TY, kPooled>), grid, block, 0, st,
+                           jobs, items, n_items, total_tiles, chunk_log2);
+    else
+        hipLaunchKernelGGL((pm_step_kernel<NT, ST, STORE, TX, TY, kFormPlain>), grid, block, 0, st,
+                           jobs, items, n_items, total_tiles, chunk_log2);
     return hipGetLastError();
 }
 
 // 256-lane tiles of four shapes and two 128-lane tiles (finer granularity
-// for small views).  Variants that force more waves per SIMD than the
-// register budget allows spill to scratch and are not offered.
+// for small views).  No variant asks for waves (wpe 1); kStepWaves does so for
+// the windows that need it, in every variant alike.
 const StepVariant kStepVariants[] = {
     {16, 16, 1}, {32, 8, 1}, {8, 32, 1}, {64, 4, 1}, {32, 4, 1}, {16, 8, 1},
 };
@@ -383,17 +417,17 @@ const int kNumStepVariants = (int)(sizeof(kStepVariants) / sizeof(kStepVariants[
 
 template <int NT, int ST, int STORE>
 static hipError_t launch_tuned(int variant, const DevJob* jobs, const StepItem* items, int n_items,
-                               int total_tiles, hipStream_t st)
+                               int total_tiles, bool start_only, hipStream_t st)
 {
+#define HP3D_SV(V_, TX_, TY_)                                                                    \
+    case V_:                                                                                     \
+        return launch_t<NT, ST, STORE, TX_, TY_>(jobs, items, n_items, total_tiles, start_only, st);
     switch (variant) {
-        case 0: return launch_t<NT, ST, STORE, 16, 16, 1>(jobs, items, n_items, total_tiles, st);
-        case 1: return launch_t<NT, ST, STORE, 32, 8, 1>(jobs, items, n_items, total_tiles, st);
-        case 2: return launch_t<NT, ST, STORE, 8, 32, 1>(jobs, items, n_items, total_tiles, st);
-        case 3: return launch_t<NT, ST, STORE, 64, 4, 1>(jobs, items, n_items, total_tiles, st);
-        case 4: return launch_t<NT, ST, STORE, 32, 4, 1>(jobs, items, n_items, total_tiles, st);
-        case 5: return launch_t<NT, ST, STORE, 16, 8, 1>(jobs, items, n_items, total_tiles, st);
+        HP3D_SV(0, 16, 16) HP3D_SV(1, 32, 8) HP3D_SV(2, 8, 32) HP3D_SV(3, 64, 4)
+        HP3D_SV(4, 32, 4) HP3D_SV(5, 16, 8)
         default: return hipErrorInvalidValue;
     }
+#undef HP3D_SV
 }
 
 bool step_variant_tunable(int radius, int stride) { return radius == 5; }
@@ -402,18 +436,19 @@ int step_tile_tx(int variant) { return kStepVariants[variant].tx; }
 int step_tile_ty(int variant) { return kStepVariants[variant].ty; }
 
 hipError_t launch_step(int store, int radius, int stride, int variant, const DevJob* jobs,
-                       const StepItem* items, int n_items, int total_tiles, hipStream_t st)
+                       const StepItem* items, int n_items, int total_tiles, bool start_only,
+                       hipStream_t st)
 {
     if (variant < 0 || variant >= kNumStepVariants) return hipErrorInvalidValue;
     if (!step_variant_tunable(radius, stride) && variant != 0) return hipErrorInvalidValue;
 #define HP3D_TUNED(R_, S_, ST_)                                                                  \
     if (radius == R_ && stride == S_ && store == ST_)                                           \
         return launch_tuned<(2 * R_) / S_ + 1, S_, ST_>(variant, jobs, items, n_items, total_tiles, \
-                                                        st);
+                                                        start_only, st);
 #define HP3D_PLAIN(R_, S_, ST_)                                                                 \
     if (radius == R_ && stride == S_ && store == ST_)                                          \
-        return launch_t<(2 * R_) / S_ + 1, S_, ST_, 16, 16, 1>(jobs, items, n_items, total_tiles, \
-                                                                st);
+        return launch_t<(2 * R_) / S_ + 1, S_, ST_, 16, 16>(jobs, items, n_items, total_tiles,  \
+                                                             start_only, st);
     HP3D_TUNED(5, 1, kStoreF32) HP3D_TUNED(5, 2, kStoreF32)
     HP3D_TUNED(5, 1, kStoreF16) HP3D_TUNED(5, 2, kStoreF16)
     HP3D_PLAIN(1, 1, kStoreF32) HP3D_PLAIN(2, 1, kStoreF32) HP3D_PLAIN(3, 1, kStoreF32)

@@ -274,7 +274,8 @@ int hp3d_pm_batch_run(hp3d_pm_ctx* ctx, const hp3d_view_desc* descs, int n,
 #define HP3D_PM_NUM_VARIANTS 6
 int hp3d_pm_autotune(hp3d_pm_ctx* ctx, const hp3d_view_desc* descs, int n, int* best_variant,
                      float* times_ms);
-/* Tile shape and waves-per-SIMD hint of a variant. */
+/* Tile shape of a variant and the waves per SIMD that it asks the compiler for (a
+ * window whose registers would hold fewer than 4 asks for 4 in every variant). */
 int hp3d_pm_variant_info(int variant, int* tile_cols, int* tile_rows, int* waves_per_simd);
 /* Persist / restore the autotuner's choices (text, one line per key). */
 int hp3d_pm_tune_save(const hp3d_pm_ctx* ctx, const char* path);

@@ -75,3 +75,19 @@ def test_view_kernels_fit_four_waves_without_spills(kernels, name):
     for k, v in ks.items():
         assert v[".vgpr_spill_count"] == 0, (k, v[".vgpr_spill_count"])
         assert v[".vgpr_count"] <= 128, (k, v[".vgpr_count"])
+
+
+# forms of pm_step.hip: plain, pooled, start only
+SPILL = {("11", "1", "0", "1"), ("7", "1", "0", "1"), ("7", "1", "1", "1")}
+
+
+def test_step_kernels_fit_four_waves_and_spill_only_where_stated(kernels):
+    ks = of(kernels, "pm_step_kernel")
+    seen = set()
+    for k, v in ks.items():
+        nt, st, store, _, _, form = re.findall(r"-?\d+", k.split("<")[1])
+        assert v[".vgpr_count"] <= 128, (k, v[".vgpr_count"])
+        if v[".vgpr_spill_count"]:
+            seen.add((nt, st, store, form))
+            assert v[".vgpr_spill_count"] <= 16, k
+    assert seen <= SPILL, seen - SPILL
