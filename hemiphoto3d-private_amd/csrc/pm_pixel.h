@@ -309,6 +309,7 @@ __device__ __forceinline__ WinRef window_ref_sums(const float* __restrict__ lwin
 // taps, FP32: 0.48 against 0.51 ms a colour).
 template <int NT> constexpr int kPassChunk = NT <= 7 ? NT : (NT + 1) / 2;
 template <int NT> constexpr int kCostChunk = NT;
+constexpr int kOutsideTaps = 4;   // taps a row from which source_cost tests window_outside
 
 // The window's taps for one candidate and source (patchmatch_mvs.cu:273-307).
 // MASKED = false is used only when every tap is known to be inside the image;
@@ -601,8 +602,11 @@ __device__ __forceinline__ float source_cost(const DevView& v, int s,
     // No tap of any lane's window in the image: the cost is that of no sample.
     // (9 % of the wave evaluations of a 4-source 30-degree arc, image-edge
     // bands that the outer sources do not see, otherwise run the masked loop
-    // for nothing.)
-    if (!__all(inside)) {
+    // for nothing.)  Not for windows of up to 3 taps a row, whose loop is hardly
+    // longer than the test: it took them 10 to 17 registers, with FP16 planes or
+    // 2 x 2 taps the fifth wave (two 640x480 views, 2 sources, 8 iterations, 2 x 2
+    // FP32: 0.546 ms without, 0.694 with; 3 x 3 FP16 0.666, 0.788).
+    if (NT >= kOutsideTaps && !__all(inside)) {
         bool outside = window_outside(cx, cy, cz, h00, h01, h10, h11, h20, h21, (float)R,
                                       (float)v.W, (float)v.H);
         if constexpr (kLocalCoords)

@@ -91,3 +91,12 @@ def test_step_kernels_fit_four_waves_and_spill_only_where_stated(kernels):
             seen.add((nt, st, store, form))
             assert v[".vgpr_spill_count"] <= 16, k
     assert seen <= SPILL, seen - SPILL
+
+
+@pytest.mark.parametrize("name", ["pm_halfpass_kernel", "pm_step_kernel"])
+def test_smallest_windows_fit_five_waves(kernels, name):
+    """2 x 2 taps, and 3 x 3 with FP16 planes: 96 registers."""
+    for k, v in of(kernels, name).items():
+        nt, st, store = re.findall(r"\d+", k.split("<")[1])[:3]
+        if nt == "2" or (nt == "3" and store == "1"):
+            assert v[".vgpr_count"] <= 96, (k, v[".vgpr_count"])
