@@ -322,15 +322,9 @@ static void launch_pass_t(const DevView& v, int mode, int iteration, int parity,
     constexpr int kTX = kPlainTX, kTY = kPlainTY;
     const int tiles_x = (v.Wc + kTX - 1) / kTX;
     const int tiles = tiles_x * ((v.H + kTY - 1) / kTY);
-    // LDS the kernel does not use, to hold fewer workgroups on a CU: the 121-tap
-    // initial cost, whose random hypotheses scatter the gathers, thrashes the L1
-    // with the 5 waves to a SIMD that its registers allow (FP32, 4 waves against
-    // 5: 1280x960 with 8 sources 0.584 against 0.602 ms a colour; with FP16's
-    // halved lines no difference)
-    constexpr unsigned kIdleLds = NT >= 11 && STORE == kStoreF32 ? 12288 : 0;
     if (mode == kPassCost)
         hipLaunchKernelGGL((pm_cost_kernel<NT, ST, STORE, kTX, kTY>), dim3(xcd_grid(2 * tiles)),
-                           dim3(kTX * kTY), kIdleLds, st, v, tiles_x, tiles);
+                           dim3(kTX * kTY), 0, st, v, tiles_x, tiles);
     else if (NT >= kPoolTaps && tiles >= kPoolTiles && pool_refinement(v.S, v.top_k, iteration))
         hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY, (NT >= kPoolTaps)>),
                            dim3(xcd_grid(tiles)), dim3(kTX * kTY), 0, st, v, iteration, parity,

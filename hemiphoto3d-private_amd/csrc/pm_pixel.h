@@ -225,10 +225,13 @@ template <> struct SrcImage<kStoreF32> {
     unsigned pitch;
     __device__ SrcImage(const DevView& v, int s)
         : rsrc(make_rsrc(v.src_coef[s], v.coef_bytes / 8, 8)), pitch((unsigned)v.pitch_plain) {}
-    __device__ __forceinline__ Quad load(int ix, int iy, bool ok = true) const
+    __device__ __forceinline__ unsigned index(int ix, int iy, bool ok) const
     {
-        unsigned idx = __umul24((unsigned)iy, pitch) + (unsigned)ix;
-        idx = ok ? idx : kIdxNowhere;
+        const unsigned idx = __umul24((unsigned)iy, pitch) + (unsigned)ix;
+        return ok ? idx : kIdxNowhere;
+    }
+    __device__ __forceinline__ Quad load(unsigned idx) const
+    {
         return __builtin_bit_cast(float4, struct_load_b128(rsrc, (int)idx, 0, 0, 0));
     }
     static __device__ __forceinline__ float lerp(const Quad& q, float au, float aw)
@@ -243,10 +246,13 @@ template <> struct SrcImage<kStoreF16> {
     unsigned pitch;
     __device__ SrcImage(const DevView& v, int s)
         : rsrc(make_rsrc(v.src_coef[s], v.coef_bytes / 4, 4)), pitch((unsigned)v.pitch_plain) {}
-    __device__ __forceinline__ Quad load(int ix, int iy, bool ok = true) const
+    __device__ __forceinline__ unsigned index(int ix, int iy, bool ok) const
     {
-        unsigned idx = __umul24((unsigned)iy, pitch) + (unsigned)ix;
-        idx = ok ? idx : kIdxNowhere;
+        const unsigned idx = __umul24((unsigned)iy, pitch) + (unsigned)ix;
+        return ok ? idx : kIdxNowhere;
+    }
+    __device__ __forceinline__ Quad load(unsigned idx) const
+    {
         return __builtin_bit_cast(half4_t, struct_load_b64(rsrc, (int)idx, 0, 0, 0));
     }
     static __device__ __forceinline__ float lerp(const Quad& q, float au, float aw)
@@ -302,11 +308,11 @@ __device__ __forceinline__ WinRef window_ref_sums(const float* __restrict__ lwin
 // registers for) that kernel held 167 registers and 3 waves to a SIMD, its
 // unrolled loops filled more than the 64 KiB instruction cache, and a change
 // anywhere else could make it wait for each gather by itself (+23 % time); in
-// chunks it holds 119, 4 waves, and every loop is one row long: 1280x960 with 8
-// sources at stride 1, FP32, 2.00 -> 1.94 ms a half-pass.
+// chunks it holds 123 (FP16 111), 4 waves, and every loop is one row long: 1280x960
+// with 8 sources at stride 1, FP32, 2.00 -> 1.94 ms a half-pass.
 // Initial cost: whole rows.  Its random hypotheses scatter the gathers, the
-// L1's line rate bounds it, and chunks only add to its waits (1600x1200, 11x11
-// taps, FP32: 0.48 against 0.51 ms a colour).
+// L1's line rate bounds it, and chunks only add to its waits (1600x1200, 4 sources,
+// 11x11 taps, FP32: 0.86 against 0.92 ms).
 template <int NT> constexpr int kPassChunk = NT <= 7 ? NT : (NT + 1) / 2;
 template <int NT> constexpr int kCostChunk = NT;
 constexpr int kOutsideTaps = 4;   // taps a row from which source_cost tests window_outside
@@ -334,6 +340,15 @@ constexpr int kOutsideTaps = 4;   // taps a row from which source_cost tests win
 // (cx, cy) and the columns (h00, h10), (h01, h11) may be relative to an
 // integer base (bu, bv): the taps' coordinates are then u - bu and v - bv,
 // and the base is added back to the texel index.
+//
+// A row's neighbouring taps read the same cache lines, 64 a gather where the
+// hypotheses are random, and the L1 holds four gathers' worth: the row's gathers
+// have to come back to back, before other waves' push those lines out.  The
+// compiler does that by itself but in the masked loop of 11 FP32 quads (kBurst),
+// where it put 13 instructions of address arithmetic between any two: initial
+// cost, 11 x 11 taps, 2400x1800, 6 sources, 3.80 ms, against 3.01 with all
+// addresses first (with 3 waves to a SIMD instead of 4, 3.49 and 3.01);
+// 3200x2400, 3 sources, 3.30 and 2.79; 1600x1200, 4 sources, 0.93 and 0.86.
 template <int NT, int ST, int STORE, bool MASKED, bool ZCHK, int C>
 __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
                                            const float* __restrict__ lwin, int lp, float cx,
@@ -358,7 +373,10 @@ __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
         const float* lrow = lwin + j * ST * lp;
 #pragma unroll
         for (int i0 = 0; i0 < NT; i0 += C) {
+            constexpr bool kBurst = MASKED && C >= 11 && STORE == kStoreF32;
+            static_assert(!kBurst || C == NT, "whole rows");
             typename SrcImage<STORE>::Quad q[C];
+            unsigned idx[C];
             float au[C], aw[C], rv[C];
             bool okv[C];
 #pragma unroll
@@ -381,8 +399,19 @@ __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
                 // invalid tap's load goes nowhere and reads zeros (so sval = 0)
                 okv[t] = !MASKED || ((!ZCHK || fabsf(wz) >= 1e-8f) & ((unsigned)ix <= umax) &
                                      ((unsigned)iy <= vmax));
-                q[t] = img.load(ix, iy, okv[t]);
-                rv[t] = lrow[i * ST];
+                idx[t] = img.index(ix, iy, okv[t]);
+                if (!kBurst) {
+                    q[t] = img.load(idx[t]);
+                    rv[t] = lrow[i * ST];
+                }
+            }
+            if (kBurst) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < C; ++t) q[t] = img.load(idx[t]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < C; ++t) rv[t] = lrow[(t + F < NT ? t + F : t + F - NT) * ST];
             }
 #pragma unroll
             for (int t = 0; t < C; ++t) {

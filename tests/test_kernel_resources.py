@@ -100,3 +100,27 @@ def test_smallest_windows_fit_five_waves(kernels, name):
         nt, st, store = re.findall(r"\d+", k.split("<")[1])[:3]
         if nt == "2" or (nt == "3" and store == "1"):
             assert v[".vgpr_count"] <= 96, (k, v[".vgpr_count"])
+
+
+def test_initial_cost_issues_a_rows_gathers_together(tmp_path):
+    """11 x 11 FP32: the 11 gathers of a row come with no vector arithmetic between
+    them, in the masked and in the plain tap loop."""
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    with open(LIB, "rb") as f:
+        blob = f.read()
+    for elf in code_objects(blob):
+        name = [k[".name"] for k in metadata(elf) if "pm_cost_kernelILi11ELi1ELi0E" in k[".name"]]
+        if name:
+            break
+    path = tmp_path / "k.elf"
+    path.write_bytes(elf)
+    text = subprocess.run([objdump, "-d", "--no-show-raw-insn", f"--disassemble-symbols={name[0]}",
+                           str(path)], capture_output=True, text=True, check=True).stdout
+    ops = re.findall(r"^\s+([a-z]\w+)", text, re.M)
+    gathers = [i for i, op in enumerate(ops) if op == "buffer_load_dwordx4"]
+    assert len(gathers) == 22
+    for row in (gathers[:11], gathers[11:]):
+        between = [op for op in ops[row[0]:row[-1]] if op.startswith("v_")]
+        assert len(between) <= 2, between
