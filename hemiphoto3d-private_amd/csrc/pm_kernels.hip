@@ -269,6 +269,22 @@ constexpr int kPlainTX = HP3D_PLAIN_TX, kPlainTY = HP3D_PLAIN_TY;
 constexpr int kPlainTX = 32, kPlainTY = 8;
 #endif
 
+// Whether a half-pass of `tiles` tiles takes `halves` of half the height instead:
+// where the workgroups of the fullest CU then hold less of the view.  Every tile is
+// in flight at once here (4 workgroups to a CU), and the launch is as long as the
+// fullest CU's share: 640x480 has 600 tiles, at most 3 to a CU, against 1200 halves,
+// at most 5 (half-passes of the first iteration, 2 sources, 11 x 11 taps: FP32 0.281
+// ms as tiles, 0.241 as halves, FP16 0.266 and 0.237; 680x510, 704 or 1408, 3 or 6:
+// 0.289 and 0.301).  In the first two iterations: later their shorter lists cost more
+// (480x360, 1 source, FP32: the first two 0.029 ms faster, the next six 0.052 slower).
+// Not for smaller windows, nor for 9 x 9 FP16, which gained 9 % in its first
+// iteration and lost 3 % in eight.
+constexpr int kCUs = 256, kHalfIterations = 2;
+static bool halve_tiles(int tiles, int halves)
+{
+    return (halves + kCUs - 1) / kCUs < 2 * ((tiles + kCUs - 1) / kCUs);
+}
+
 // The split kernels' tile: 16 x 4 (32 x 4 pixels; 32x2 and 8x8 within 3 %).
 constexpr int kSplitTX = 16, kSplitTY = 4;
 
@@ -322,6 +338,9 @@ static void launch_pass_t(const DevView& v, int mode, int iteration, int parity,
     constexpr int kTX = kPlainTX, kTY = kPlainTY;
     const int tiles_x = (v.Wc + kTX - 1) / kTX;
     const int tiles = tiles_x * ((v.H + kTY - 1) / kTY);
+    constexpr bool kHalf = (NT >= 11 || (NT >= 9 && STORE == kStoreF32)) && kTX * kTY % 128 == 0;
+    constexpr int kHalfTY = kHalf ? kTY / 2 : kTY;
+    const int halves = tiles_x * ((v.H + kHalfTY - 1) / kHalfTY);
     if (mode == kPassCost)
         hipLaunchKernelGGL((pm_cost_kernel<NT, ST, STORE, kTX, kTY>), dim3(xcd_grid(2 * tiles)),
                            dim3(kTX * kTY), 0, st, v, tiles_x, tiles);
@@ -329,6 +348,11 @@ static void launch_pass_t(const DevView& v, int mode, int iteration, int parity,
         hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY, (NT >= kPoolTaps)>),
                            dim3(xcd_grid(tiles)), dim3(kTX * kTY), 0, st, v, iteration, parity,
                            pass_seed, tiles_x, tiles);
+    else if (kHalf && tiles < kPoolTiles && iteration < v.first_iteration + kHalfIterations &&
+             halve_tiles(tiles, halves))
+        hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kHalfTY, false>),
+                           dim3(xcd_grid(halves)), dim3(kTX * kHalfTY), 0, st, v, iteration, parity,
+                           pass_seed, tiles_x, halves);
     else
         hipLaunchKernelGGL((pm_halfpass_kernel<NT, ST, STORE, kTX, kTY, false>),
                            dim3(xcd_grid(tiles)), dim3(kTX * kTY), 0, st, v, iteration, parity,
