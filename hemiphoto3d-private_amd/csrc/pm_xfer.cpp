@@ -2,6 +2,7 @@
 #include "pm_xfer.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <new>
 #include <system_error>
@@ -186,7 +187,8 @@ void HostLink::worker()
         ++inside_;
         lk.unlock();
         came_.store(true, std::memory_order_relaxed);
-        // tasks come every few microseconds while a copy is on: no sleeping
+        // tasks come every few microseconds while a copy is on: no sleeping (and
+        // where it has to wait for its stream, slot_ready ends this)
         while (active_.load(std::memory_order_acquire))
             if (!work_one()) std::this_thread::yield();
         lk.lock();
@@ -218,7 +220,7 @@ void HostLink::hand_out(size_t piece)
     ready_.store((piece + 1) * kTasks, std::memory_order_release);
 }
 
-// Finishes the handed-out tasks; no worker touches the pieces any more on return.
+// Finishes the handed-out tasks; no worker touches the pieces on return (until wake()).
 void HostLink::end()
 {
     while (work_one()) {}
@@ -230,11 +232,29 @@ void HostLink::end()
     cv_.wait(lk, [&] { return inside_ == 0; });
 }
 
+// The copy out of the slot, over on return.  While copies follow each other that takes
+// tens of microseconds; where it takes longer, the stream is still at the work before
+// them (an earlier view's passes), and the threads sleep until it has come.
 hipError_t HostLink::slot_ready(int slot)
 {
     if (!in_flight_[slot]) return hipSuccess;
     in_flight_[slot] = false;
-    return hipEventSynchronize(ev_[slot]);
+    const auto patience = std::chrono::steady_clock::now() + std::chrono::microseconds(kPatienceUs);
+    hipError_t e;
+    while ((e = hipEventQuery(ev_[slot])) == hipErrorNotReady) {
+        (void)hipGetLastError();   // an answer here, not an error
+        if (std::chrono::steady_clock::now() < patience) {
+            help();
+            continue;
+        }
+        const bool awake = active_.load(std::memory_order_relaxed);
+        if (awake) end();
+        e = hipEventSynchronize(ev_[slot]);
+        came_.store(false, std::memory_order_relaxed);
+        if (awake) wake();
+        break;
+    }
+    return e;
 }
 
 hipError_t HostLink::download(const std::vector<Seg>& segs, hipStream_t st)

@@ -60,6 +60,7 @@ private:
         return total < (4u << 20) ? 1u << 20 : total < (24u << 20) ? 2u << 20 : kSlotBytes;
     }
     static constexpr int kTasks = 4;       // a piece's shares among the threads
+    static constexpr int kPatienceUs = 300;   // a 4 MiB piece takes 75 us, waking threads 50
     static constexpr int kMaxParts = 4;
     static constexpr int kMaxWorkers = 6;
 
