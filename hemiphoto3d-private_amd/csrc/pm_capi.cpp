@@ -32,6 +32,8 @@ int hp3d_pm_ctx::fail(int code, const char* fmt, ...)
 
 int hp3d_pm_ctx::hip_fail(hipError_t e, const char* what)
 {
+    // reported here: not again by the next launch's check of the last error
+    (void)hipGetLastError();
     return fail(HP3D_ERR_DEVICE, "%s: %s", what, hipGetErrorString(e));
 }
 

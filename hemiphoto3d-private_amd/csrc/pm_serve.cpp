@@ -518,6 +518,7 @@ int hp3d_server_create(const hp3d_server_opts* opts, hp3d_pm_server** out)
              hipHostMalloc((void**)&s->h_items[b], opts->max_jobs * sizeof(StepItem)) == hipSuccess &&
              hipEventCreate(&s->ev_a[b]) == hipSuccess && hipEventCreate(&s->ev_b[b]) == hipSuccess;
     if (!ok) {
+        (void)hipGetLastError();   // reported here, not by this thread's next launch
         hp3d_server_destroy(s.release());
         return HP3D_ERR_DEVICE;
     }
