@@ -83,14 +83,14 @@ __global__ __launch_bounds__(kFuseBlock) void fuse_count_kernel(const FuseViewDe
     }
 }
 
-// Exclusive scan of n block counts (one workgroup; n is at most a few hundred
-// thousand), total into *total.
-__global__ __launch_bounds__(1024) void fuse_scan_kernel(const int* counts, int n,
+// Exclusive scan of n block counts from `base` on (one workgroup; n is at most a few
+// hundred thousand), its end into *total.
+__global__ __launch_bounds__(1024) void fuse_scan_kernel(const int* counts, int n, long long base,
                                                          long long* offsets, long long* total)
 {
     __shared__ long long carry;
     __shared__ long long part[1024 / 64];
-    if (threadIdx.x == 0) carry = 0;
+    if (threadIdx.x == 0) carry = base;
     __syncthreads();
     for (int start = 0; start < n; start += 1024) {
         const int i = start + threadIdx.x;
@@ -192,34 +192,24 @@ __global__ __launch_bounds__(kFuseBlock) void fuse_write_kernel(const FuseViewDe
     }
 }
 
-}  // namespace
+size_t a256(size_t b) { return (b + 255) & ~(size_t)255; }
+size_t fuse_blocks(size_t px) { return (px + kFuseSpan - 1) / kFuseSpan; }
 
-}  // namespace hp3d
-
-using namespace hp3d;
-
-extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n,
-                            float min_confidence, float* positions, float* normals,
-                            float* colors, size_t capacity, size_t* count)
+// One attempt at hp3d_pm_fuse, its arguments checked.  All views at once, or
+// (one_by_one) count, scan and write view after view, which takes less memory for
+// the view table, counts and offsets.  *refused: the memory was not to be had.
+int fuse_views(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n, float min_confidence,
+               float* positions, float* normals, float* colors, size_t capacity, size_t* count,
+               bool one_by_one, bool* refused)
 {
-    if (!ctx) return HP3D_ERR_INVALID_ARG;
-    if (!views || n < 1 || !count || !(min_confidence == min_confidence))
-        return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: bad arguments");
-    for (int i = 0; i < n; ++i) {
-        const hp3d_fuse_view& v = views[i];
-        if (v.width < 1 || v.height < 1 || !v.depth ||
-            (long long)v.width * v.height > (1ll << 31) - kFuseBlock ||
-            (v.color && v.color_channels != 1 && v.color_channels != 3))
-            return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: view %d is malformed", i);
-    }
-    (void)hipSetDevice(ctx->device);
+    *refused = false;
     // what the call needs on the device: to count, depth and confidence; to
-    // write, the maps of what it writes.  One device block: the maps, the views, counts, offsets.
+    // write, the maps of what it writes.  One device block: the maps, then the total,
+    // the views, offsets and counts.
     const bool write = positions != nullptr;
-    auto a256 = [](size_t b) { return (b + 255) & ~(size_t)255; };
     std::vector<FuseViewDev> g(n);
     std::vector<HostLink::Seg> segs;   // device: offsets into the block, for now
-    size_t total = 0, blocks = 0;
+    size_t total = 0, blocks = 0, largest = 0;
     auto put = [&](const void* host, size_t bytes) {
         const size_t off = total;
         segs.push_back({const_cast<void*>(host), reinterpret_cast<void*>(off), bytes});
@@ -242,27 +232,31 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
         d.H = v.height;
         d.channels = v.color ? v.color_channels : 0;
         d.min_conf = min_confidence;
-        d.first_block = (int)blocks;
+        d.first_block = one_by_one ? 0 : (int)blocks;
         off[i].depth = put(v.depth, px * 4);
         if (v.confidence) off[i].conf = put(v.confidence, px * 4);
         if (write && normals && v.normal) off[i].normal = put(v.normal, px * 12);
         if (write && colors && v.color) off[i].color = put(v.color, px * v.color_channels);
-        blocks += (px + kFuseSpan - 1) / kFuseSpan;
+        blocks += fuse_blocks(px);
+        largest = std::max(largest, fuse_blocks(px));
     }
-    if (blocks > 0x7fffffff)
-        return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: %zu blocks of pixels", blocks);
-    const size_t views_off = put(g.data(), n * sizeof(FuseViewDev));
-    const size_t counts_off = total;
-    total += a256(blocks * 4) + a256(blocks * 8) + 256;
+    // (view by view, less than a total, offsets and counts of 256-pixel blocks take)
+    const size_t held = one_by_one ? 1 : n, rows = one_by_one ? largest : blocks;
+    const size_t scratch = total;
+    const size_t offsets_off = scratch + 8 + held * sizeof(FuseViewDev);
+    static_assert(sizeof(FuseViewDev) % 8 == 0, "offsets aligned after the views");
+    total += a256(8 + held * sizeof(FuseViewDev) + rows * 12);
     void* block = nullptr;
     int rc = ctx->dev_alloc(&block, total, "fusion maps");
-    if (rc) return rc;
+    if (rc) {
+        *refused = true;
+        return rc;
+    }
     char* base = static_cast<char*>(block);
-    const FuseViewDev* d_views = reinterpret_cast<const FuseViewDev*>(base + views_off);
-    int* d_counts = reinterpret_cast<int*>(base + counts_off);
-    long long* d_offsets = reinterpret_cast<long long*>(base + counts_off + a256(blocks * 4));
-    long long* d_total = reinterpret_cast<long long*>(base + counts_off + a256(blocks * 4) +
-                                                      a256(blocks * 8));
+    long long* d_total = reinterpret_cast<long long*>(base + scratch);
+    FuseViewDev* d_views = reinterpret_cast<FuseViewDev*>(base + scratch + 8);
+    long long* d_offsets = reinterpret_cast<long long*>(base + offsets_off);
+    int* d_counts = reinterpret_cast<int*>(base + offsets_off + rows * 8);
     for (auto& s : segs) s.dev = base + reinterpret_cast<size_t>(s.dev);
     for (int i = 0; i < n; ++i) {
         const hp3d_fuse_view& v = views[i];
@@ -271,22 +265,35 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
         if (write && normals && v.normal) g[i].normal = reinterpret_cast<const float*>(base + off[i].normal);
         if (write && colors && v.color) g[i].color = reinterpret_cast<const uint8_t*>(base + off[i].color);
     }
+    if (!one_by_one) segs.push_back({g.data(), d_views, n * sizeof(FuseViewDev)});
     hipError_t e = ctx->link.upload(segs, ctx->stream);
-    long long npts_l = 0;
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(fuse_count_kernel, dim3((unsigned)blocks), dim3(kFuseBlock), 0,
-                           ctx->stream, d_views, n, d_counts);
+    // the views of group k, their blocks, and the ranks of their points from `from` on
+    const int groups = one_by_one ? n : 1, group_views = one_by_one ? 1 : n;
+    auto group_blocks = [&](int k) {
+        return one_by_one ? fuse_blocks((size_t)g[k].W * g[k].H) : blocks;
+    };
+    auto rank = [&](int k, long long from) -> hipError_t {
+        if (one_by_one) {
+            const hipError_t ue = ctx->link.upload({{&g[k], d_views, sizeof(FuseViewDev)}}, ctx->stream);
+            if (ue != hipSuccess) return ue;
+        }
+        hipLaunchKernelGGL(fuse_count_kernel, dim3((unsigned)group_blocks(k)), dim3(kFuseBlock), 0,
+                           ctx->stream, d_views, group_views, d_counts);
         hipLaunchKernelGGL(fuse_scan_kernel, dim3(1), dim3(1024), 0, ctx->stream, d_counts,
-                           (int)blocks, d_offsets, d_total);
-        e = hipGetLastError();
+                           (int)group_blocks(k), from, d_offsets, d_total);
+        return hipGetLastError();
+    };
+    std::vector<long long> from(groups + 1, 0);
+    for (int k = 0; k < groups && e == hipSuccess; ++k) {
+        e = rank(k, from[k]);
+        if (e == hipSuccess) e = ctx->link.download({{&from[k + 1], d_total, sizeof(long long)}}, ctx->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     }
-    if (e == hipSuccess) e = ctx->link.download({{&npts_l, d_total, sizeof npts_l}}, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
         ctx->dev_free(block, total);
         return ctx->hip_fail(e, "fusion count");
     }
-    const size_t npts = (size_t)npts_l;
+    const size_t npts = (size_t)from[groups];
     *count = npts;
     if (!positions || npts == 0) {
         ctx->dev_free(block, total);
@@ -304,14 +311,19 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
     rc = ctx->dev_alloc(&out, per * nbuf, "fusion output");
     if (rc) {
         ctx->dev_free(block, total);
+        *refused = true;
         return rc;
     }
     float* d_pos = static_cast<float*>(out);
     float* d_nrm = normals ? d_pos + 3 * npts : nullptr;
     float* d_col = colors ? d_pos + 3 * npts * (normals ? 2 : 1) : nullptr;
-    hipLaunchKernelGGL(fuse_write_kernel, dim3((unsigned)blocks), dim3(kFuseBlock), 0, ctx->stream,
-                       d_views, n, d_offsets, d_pos, d_nrm, d_col);
-    e = hipGetLastError();
+    for (int k = 0; k < groups && e == hipSuccess; ++k) {
+        if (one_by_one) e = rank(k, from[k]);
+        if (e != hipSuccess) break;
+        hipLaunchKernelGGL(fuse_write_kernel, dim3((unsigned)group_blocks(k)), dim3(kFuseBlock), 0,
+                           ctx->stream, d_views, group_views, d_offsets, d_pos, d_nrm, d_col);
+        e = hipGetLastError();
+    }
     segs.assign({{positions, d_pos, per}});
     if (normals) segs.push_back({normals, d_nrm, per});
     if (colors) segs.push_back({colors, d_col, per});
@@ -321,4 +333,40 @@ extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n
     ctx->dev_free(block, total);
     if (e != hipSuccess) return ctx->hip_fail(e, "fusion");
     return HP3D_OK;
+}
+
+}  // namespace
+
+}  // namespace hp3d
+
+using namespace hp3d;
+
+extern "C" int hp3d_pm_fuse(hp3d_pm_ctx* ctx, const hp3d_fuse_view* views, int n,
+                            float min_confidence, float* positions, float* normals,
+                            float* colors, size_t capacity, size_t* count)
+{
+    if (!ctx) return HP3D_ERR_INVALID_ARG;
+    if (!views || n < 1 || !count || !(min_confidence == min_confidence))
+        return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: bad arguments");
+    size_t blocks = 0;
+    for (int i = 0; i < n; ++i) {
+        const hp3d_fuse_view& v = views[i];
+        if (v.width < 1 || v.height < 1 || !v.depth ||
+            (long long)v.width * v.height > (1ll << 31) - kFuseBlock ||
+            (v.color && v.color_channels != 1 && v.color_channels != 3))
+            return ctx->fail(HP3D_ERR_INVALID_ARG, "fuse: view %d is malformed", i);
+        blocks += fuse_blocks((size_t)v.width * v.height);
+    }
+    (void)hipSetDevice(ctx->device);
+    // all views at once, unless a launch cannot hold them (2^32 threads) or their
+    // table and counts are what does not fit
+    bool refused = blocks >= 0xffffffffull / kFuseBlock;
+    int rc = HP3D_OK;
+    if (!refused)
+        rc = fuse_views(ctx, views, n, min_confidence, positions, normals, colors, capacity, count,
+                        false, &refused);
+    if (refused)
+        rc = fuse_views(ctx, views, n, min_confidence, positions, normals, colors, capacity, count,
+                        true, &refused);
+    return rc;
 }
