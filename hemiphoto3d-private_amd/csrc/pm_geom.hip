@@ -222,7 +222,9 @@ extern "C" int hp3d_pm_geom_filter(hp3d_pm_ctx* ctx, hp3d_geom_view* views, int 
         segs.push_back({views[i].depth, dptr(i, 0), px});
         if (views[i].confidence) segs.push_back({views[i].confidence, dptr(i, 4), px});
     }
-    std::vector<int> kept(retained && d_kept ? tile_base[n] : 0);
+    // (the kernel's counts are each view's own; where views share host memory, the
+    // bytes that stay are the later one's and are counted there)
+    std::vector<int> kept(retained && d_kept && !HostLink::overlap(segs) ? tile_base[n] : 0);
     if (!kept.empty()) segs.push_back({kept.data(), d_kept, kept.size() * sizeof(int)});
     if (e == hipSuccess) e = ctx->link.download(segs, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -231,7 +233,7 @@ extern "C" int hp3d_pm_geom_filter(hp3d_pm_ctx* ctx, hp3d_geom_view* views, int 
     if (retained)
         for (int i = 0; i < n; ++i) {
             int r = 0;
-            if (d_kept) {
+            if (!kept.empty()) {
                 for (size_t t = tile_base[i]; t < tile_base[i + 1] && filtered[i]; ++t) r += kept[t];
             } else {
                 const size_t px = (size_t)views[i].width * views[i].height;

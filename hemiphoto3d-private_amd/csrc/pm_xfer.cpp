@@ -24,7 +24,9 @@ bool known_to_runtime(const void* p)
     return a.type != hipMemoryTypeUnregistered;
 }
 
-bool overlap(const std::vector<HostLink::Seg>& segs)
+}  // namespace
+
+bool HostLink::overlap(const std::vector<Seg>& segs)
 {
     if (segs.size() < 2) return false;
     std::vector<std::pair<const char*, size_t>> r;
@@ -34,8 +36,6 @@ bool overlap(const std::vector<HostLink::Seg>& segs)
         if (r[i - 1].first + r[i - 1].second > r[i].first) return true;
     return false;
 }
-
-}  // namespace
 
 bool HostLink::open()
 {

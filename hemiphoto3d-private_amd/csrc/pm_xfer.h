@@ -44,6 +44,8 @@ public:
     // Host to device on st.  Returns when pageable sources are read; page-locked
     // ones are once st is synchronised.
     hipError_t upload(const std::vector<Seg>& segs, hipStream_t st);
+    // Whether segments share host memory.
+    static bool overlap(const std::vector<Seg>& segs);
     // Waits for the ring's copies and gives everything back.
     void close();
 
