@@ -224,7 +224,7 @@ extern "C" int hp3d_pm_geom_filter(hp3d_pm_ctx* ctx, hp3d_geom_view* views, int 
     }
     // (the kernel's counts are each view's own; where views share host memory, the
     // bytes that stay are the later one's and are counted there)
-    std::vector<int> kept(retained && d_kept && !HostLink::overlap(segs) ? tile_base[n] : 0);
+    std::vector<int> kept(retained && d_kept && !HostLink::overlap(segs.data(), segs.size()) ? tile_base[n] : 0);
     if (!kept.empty()) segs.push_back({kept.data(), d_kept, kept.size() * sizeof(int)});
     if (e == hipSuccess) e = ctx->link.download(segs, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);

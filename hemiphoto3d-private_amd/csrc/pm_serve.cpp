@@ -474,10 +474,10 @@ void hp3d_pm_server::complete_loop()
         }
         hipError_t e = hipEventSynchronize(j->last_ev);
         const size_t px = (size_t)j->d.width * j->d.height * 4;
-        std::vector<HostLink::Seg> segs{{j->d.out_depth, j->dj.out_depth, px}};
-        if (j->d.out_normal) segs.push_back({j->d.out_normal, j->dj.out_normal, 3 * px});
-        if (j->d.out_cost) segs.push_back({j->d.out_cost, j->dj.out_cost, px});
-        if (e == hipSuccess) e = link.download(segs, copy);
+        const HostLink::Seg segs[3] = {{j->d.out_depth, j->dj.out_depth, px},
+                                       {j->d.out_normal, j->dj.out_normal, j->d.out_normal ? 3 * px : 0},
+                                       {j->d.out_cost, j->dj.out_cost, j->d.out_cost ? px : 0}};
+        if (e == hipSuccess) e = link.download(segs, 3, copy);
         if (e == hipSuccess) e = hipStreamSynchronize(copy);
         std::lock_guard<std::mutex> lk(mu);
         if (e != hipSuccess) last_error = hipGetErrorString(e);

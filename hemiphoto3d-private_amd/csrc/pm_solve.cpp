@@ -82,16 +82,17 @@ int emit_outputs(hp3d_pm_ctx* ctx, const DevView& v, float* depth, float* normal
     for (int q = 0; q < 4; ++q) total += host[q] ? count[q] : 0;
     int rc = ctx->grow(ctx->out_stage, total * sizeof(float), "output staging");
     if (rc) return rc;
-    std::vector<HostLink::Seg> segs;
+    HostLink::Seg segs[4];
+    int n_segs = 0;
     float* p = static_cast<float*>(ctx->out_stage.ptr);
     for (int q = 0; q < 4; ++q) {
         if (!host[q]) continue;
         dev[q] = p;
-        segs.push_back({host[q], p, count[q] * sizeof(float)});
+        segs[n_segs++] = {host[q], p, count[q] * sizeof(float)};
         p += count[q];
     }
     e = launch_finalize(v, dev[0], dev[1], dev[2], dev[3], ctx->stream);
-    if (e == hipSuccess) e = ctx->link.download(segs, ctx->stream);
+    if (e == hipSuccess) e = ctx->link.download(segs, n_segs, ctx->stream);
     return e == hipSuccess ? HP3D_OK : ctx->hip_fail(e, "output copy");
 }
 
@@ -275,10 +276,11 @@ int solve_views(hp3d_pm_ctx* ctx, int n, const hp3d_view_desc* d, const Image* c
             float* dst[4] = {out[j].depth, out[j].normal, out[j].cost, out[j].confidence};
             const size_t cnt[4] = {px, 3 * px, px, px};
             e = hipStreamWaitEvent(ctx->copy_stream, ctx->ev_fin[k], 0);
-            std::vector<HostLink::Seg> segs;
+            HostLink::Seg segs[4];
+            int n_segs = 0;
             for (int q = 0; q < 4; ++q)
-                if (dst[q]) segs.push_back({dst[q], sd[k][q], cnt[q] * sizeof(float)});
-            if (e == hipSuccess) e = ctx->link.download(segs, ctx->copy_stream);
+                if (dst[q]) segs[n_segs++] = {dst[q], sd[k][q], cnt[q] * sizeof(float)};
+            if (e == hipSuccess) e = ctx->link.download(segs, n_segs, ctx->copy_stream);
             if (e == hipSuccess) e = hipEventRecord(ctx->ev_copied[k], ctx->copy_stream);
             if (e != hipSuccess) rc = ctx->hip_fail(e, "output download");
         }

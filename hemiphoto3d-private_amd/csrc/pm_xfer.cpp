@@ -26,11 +26,11 @@ bool known_to_runtime(const void* p)
 
 }  // namespace
 
-bool HostLink::overlap(const std::vector<Seg>& segs)
+bool HostLink::overlap(const Seg* segs, size_t n)
 {
-    if (segs.size() < 2) return false;
+    if (n < 2) return false;
     std::vector<std::pair<const char*, size_t>> r;
-    for (const auto& s : segs) r.emplace_back(static_cast<const char*>(s.host), s.bytes);
+    for (size_t i = 0; i < n; ++i) r.emplace_back(static_cast<const char*>(segs[i].host), segs[i].bytes);
     std::sort(r.begin(), r.end());
     for (size_t i = 1; i < r.size(); ++i)
         if (r[i - 1].first + r[i - 1].second > r[i].first) return true;
@@ -89,12 +89,13 @@ void HostLink::close()
 }
 
 // The pieces of the segments in pageable memory; the others are copied here.
-hipError_t HostLink::split(const std::vector<Seg>& segs, bool to_host, hipStream_t st)
+hipError_t HostLink::split(const Seg* segs, size_t n, bool to_host, hipStream_t st)
 {
     pieces_.clear();
     size_t total = 0;
     std::vector<const Seg*> mine;
-    for (const Seg& s : segs) {
+    for (size_t i = 0; i < n; ++i) {
+        const Seg& s = segs[i];
         if (!s.bytes) continue;
         if (known_to_runtime(s.host)) {
             const hipError_t e =
@@ -118,27 +119,38 @@ hipError_t HostLink::split(const std::vector<Seg>& segs, bool to_host, hipStream
                 p = &pieces_.back();
                 p->dev = dev + at;
             }
-            const size_t n = std::min(s->bytes - at, chunk - p->bytes);
-            p->part[p->parts++] = {host + at, p->bytes, n};
-            p->bytes += n;
-            at += n;
+            const size_t share = std::min(s->bytes - at, chunk - p->bytes);
+            p->part[p->parts++] = {host + at, p->bytes, share};
+            p->bytes += share;
+            at += share;
         }
     }
     return hipSuccess;
 }
 
-// The copy without a ring, where there is no page-locked memory to be had.
-hipError_t HostLink::plain(bool to_host, hipStream_t st)
+// The copies by the runtime alone, in order: where there is no memory for the ring,
+// page-locked, or for the lists.
+hipError_t HostLink::plain(const Seg* segs, size_t n, bool to_host, hipStream_t st)
 {
-    for (const Piece& p : pieces_)
-        for (int k = 0; k < p.parts; ++k) {
-            char* d = p.dev + p.part[k].off;
-            const hipError_t e =
-                to_host ? hipMemcpyAsync(p.part[k].host, d, p.part[k].bytes, hipMemcpyDeviceToHost, st)
-                        : hipMemcpyAsync(d, p.part[k].host, p.part[k].bytes, hipMemcpyHostToDevice, st);
-            if (e != hipSuccess) return e;
-        }
+    for (const Seg* s = segs; s != segs + n; ++s) {
+        if (!s->bytes) continue;
+        const hipError_t e =
+            to_host ? hipMemcpyAsync(s->host, s->dev, s->bytes, hipMemcpyDeviceToHost, st)
+                    : hipMemcpyAsync(s->dev, s->host, s->bytes, hipMemcpyHostToDevice, st);
+        if (e != hipSuccess) return e;
+    }
     return hipStreamSynchronize(st);
+}
+
+// The pieces that split() made, and the segments that it copied itself.
+hipError_t HostLink::through_ring(const Seg* segs, size_t n, bool to_host, hipStream_t st)
+{
+    const hipError_t e = split(segs, n, to_host, st);
+    if (e != hipSuccess || pieces_.empty()) return e;
+    if (!open()) return plain(segs, n, to_host, st);
+    if (!alone_) start_workers();
+    begin(to_host);
+    return to_host ? drain(st) : fill(st);
 }
 
 // Task i: a share of piece i / kTasks.
@@ -257,19 +269,22 @@ hipError_t HostLink::slot_ready(int slot)
     return e;
 }
 
-hipError_t HostLink::download(const std::vector<Seg>& segs, hipStream_t st)
+hipError_t HostLink::download(const Seg* segs, size_t n, hipStream_t st)
 {
-    hipError_t e = hipSuccess;
-    if (overlap(segs)) {
-        for (size_t i = 0; i < segs.size() && e == hipSuccess; ++i) e = download({segs[i]}, st);
+    try {
+        if (!overlap(segs, n)) return through_ring(segs, n, true, st);
+        hipError_t e = hipSuccess;
+        for (size_t i = 0; i < n && e == hipSuccess; ++i) e = through_ring(segs + i, 1, true, st);
         return e;
+    } catch (const std::bad_alloc&) {   // of a list: no piece is under way
+        return plain(segs, n, true, st);
     }
-    e = split(segs, true, st);
-    if (e != hipSuccess || pieces_.empty()) return e;
+}
+
+hipError_t HostLink::drain(hipStream_t st)
+{
     const size_t n = pieces_.size();
-    if (!open()) return plain(true, st);
-    if (!alone_) start_workers();
-    begin(true);
+    hipError_t e = hipSuccess;
     size_t issued = 0, handed = 0;
     while (handed < n && e == hipSuccess) {
         // keep the link busy: a copy into every free slot
@@ -306,14 +321,19 @@ hipError_t HostLink::download(const std::vector<Seg>& segs, hipStream_t st)
     return e;
 }
 
-hipError_t HostLink::upload(const std::vector<Seg>& segs, hipStream_t st)
+hipError_t HostLink::upload(const Seg* segs, size_t n, hipStream_t st)
 {
-    hipError_t e = split(segs, false, st);
-    if (e != hipSuccess || pieces_.empty()) return e;
+    try {
+        return through_ring(segs, n, false, st);
+    } catch (const std::bad_alloc&) {
+        return plain(segs, n, false, st);
+    }
+}
+
+hipError_t HostLink::fill(hipStream_t st)
+{
     const size_t n = pieces_.size();
-    if (!open()) return plain(false, st);
-    if (!alone_) start_workers();
-    begin(false);
+    hipError_t e = hipSuccess;
     if (!alone_) wake();
     size_t handed = 0, issued = 0;
     while (issued < n && e == hipSuccess) {

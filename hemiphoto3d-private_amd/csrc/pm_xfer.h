@@ -14,6 +14,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstddef>
+#include <initializer_list>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -40,12 +41,19 @@ public:
     // Device to host, after the work queued on st.  Where segments overlap in
     // host memory the later one's bytes stay.  Returns when pageable
     // destinations are written; page-locked ones are once st is synchronised.
-    hipError_t download(const std::vector<Seg>& segs, hipStream_t st);
+    hipError_t download(const Seg* segs, size_t n, hipStream_t st);
     // Host to device on st.  Returns when pageable sources are read; page-locked
     // ones are once st is synchronised.
-    hipError_t upload(const std::vector<Seg>& segs, hipStream_t st);
+    hipError_t upload(const Seg* segs, size_t n, hipStream_t st);
+    // (neither throws: without memory for their lists the runtime copies)
+
+    typedef std::initializer_list<Seg> SegList;
+    hipError_t download(SegList s, hipStream_t st) { return download(s.begin(), s.size(), st); }
+    hipError_t upload(SegList s, hipStream_t st) { return upload(s.begin(), s.size(), st); }
+    hipError_t download(const std::vector<Seg>& s, hipStream_t st) { return download(s.data(), s.size(), st); }
+    hipError_t upload(const std::vector<Seg>& s, hipStream_t st) { return upload(s.data(), s.size(), st); }
     // Whether segments share host memory.
-    static bool overlap(const std::vector<Seg>& segs);
+    static bool overlap(const Seg* segs, size_t n);
     // Waits for the ring's copies and gives everything back.
     void close();
 
@@ -75,8 +83,11 @@ private:
 
     bool open();
     void start_workers();
-    hipError_t split(const std::vector<Seg>& segs, bool to_host, hipStream_t st);
-    hipError_t plain(bool to_host, hipStream_t st);
+    hipError_t split(const Seg* segs, size_t n, bool to_host, hipStream_t st);
+    static hipError_t plain(const Seg* segs, size_t n, bool to_host, hipStream_t st);
+    hipError_t through_ring(const Seg* segs, size_t n, bool to_host, hipStream_t st);
+    hipError_t drain(hipStream_t st);
+    hipError_t fill(hipStream_t st);
     void copy_task(size_t i);
     bool work_one();
     void help();

@@ -17,6 +17,11 @@ enum hipMemoryType { hipMemoryTypeUnregistered, hipMemoryTypeHost };
 struct hipPointerAttribute_t { hipMemoryType type; };
 constexpr unsigned hipHostMallocDefault = 0, hipEventDisableTiming = 2;
 
+struct StubModel {   // the model at work: its own allocations are not the product's
+    StubModel();
+    ~StubModel();
+};
+
 struct StubStream {
     std::mutex mu;
     std::condition_variable cv;
@@ -39,6 +44,7 @@ struct StubStream {
     }};
     size_t push(std::function<void()> f)
     {
+        StubModel m;
         std::lock_guard<std::mutex> lk(mu);
         work.push_back(std::move(f));
         cv.notify_all();
@@ -108,6 +114,7 @@ inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* 
 }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
+    StubModel m;
     if (stub().refuse_host_malloc) return stub_set(hipErrorOutOfMemory);
     *p = std::malloc(n);
     std::lock_guard<std::mutex> lk(stub().mu);
@@ -123,6 +130,7 @@ inline hipError_t hipHostFree(void* p)
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
 {
+    StubModel m;
     *e = new StubEvent;
     return hipSuccess;
 }
@@ -154,6 +162,7 @@ inline hipError_t hipStreamSynchronize(hipStream_t st)
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, hipStream_t st)
 {
     const bool pinned = stub_pinned(kind == hipMemcpyHostToDevice ? s : d);
+    StubModel m;
     const size_t at = st->push([=] { std::memcpy(d, s, n); });
     ++(pinned ? stub().pinned_copies : stub().pageable_copies);
     if (!pinned) st->wait(at);   // the runtime's copy of pageable memory blocks

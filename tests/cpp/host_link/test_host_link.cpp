@@ -118,6 +118,47 @@ static bool no_ring()
     return true;
 }
 
+// Without heap memory for the lists likewise, and no exception leaves.
+static bool refuse_new = false;
+static bool no_heap()
+{
+    HostLink link;
+    StubStream st;
+    const size_t n = 100000;
+    const Bytes src = noise(n);
+    Bytes dev(n), a(n / 2), b(n - n / 2);
+    CHECK(both_ways(link, &st, 9 << 20));
+    HostLink bare;   // no ring, no threads, no lists yet
+    for (HostLink* l : {&link, &bare}) {
+        for (size_t upto = 0; upto < 2; ++upto) {
+            const HostLink::Seg up[] = {{const_cast<unsigned char*>(src.data()), dev.data(), n}};
+            const HostLink::Seg down[] = {{a.data(), dev.data(), n / 2},
+                                          {b.data(), dev.data() + n / 2, n - n / 2}};
+            std::fill(a.begin(), a.end(), 0);
+            refuse_new = true;
+            const bool ok = l->upload(up, 1, &st) == hipSuccess && l->download(down, 2, &st) == hipSuccess;
+            refuse_new = false;
+            CHECK(ok);
+            CHECK(std::memcmp(a.data(), src.data(), n / 2) == 0);
+            CHECK(std::memcmp(b.data(), src.data() + n / 2, n - n / 2) == 0);
+        }
+    }
+    return true;
+}
+// (only the calling thread's allocations are refused, not the model's streams')
+static const std::thread::id main_thread = std::this_thread::get_id();
+static thread_local int in_model = 0;
+StubModel::StubModel() { ++in_model; }
+StubModel::~StubModel() { --in_model; }
+void* operator new(size_t n)
+{
+    if (refuse_new && !in_model && std::this_thread::get_id() == main_thread) throw std::bad_alloc();
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 // An upload of more than the ring holds, behind a second of other work on its stream:
 // the copy threads sleep meanwhile.
 static bool sleeps()
@@ -148,6 +189,7 @@ int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     const bool ok = what == "sizes" ? sizes() : what == "parts" ? parts() : what == "no_ring" ? no_ring()
+                    : what == "no_heap" ? no_heap()
                     : what == "sleeps" ? sleeps() : false;
     std::puts(ok ? "ok" : "failed");
     return ok ? 0 : 1;

@@ -1,6 +1,6 @@
 """Copies through the page-locked ring (csrc/pm_xfer.cpp) on the CPU, over a model of
 the runtime calls it makes (tests/cpp/host_link): every line of its layout, pieces of
-several segments, no page-locked memory, and copy threads that sleep while an upload
+several segments, no page-locked or heap memory, and copy threads that sleep while an upload
 waits for its stream."""
 import os
 import subprocess
@@ -22,7 +22,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["sizes", "parts", "no_ring", "sleeps"])
+@pytest.mark.parametrize("check", ["sizes", "parts", "no_ring", "no_heap", "sleeps"])
 def test_host_link(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
