@@ -354,6 +354,9 @@ int hp3d_pm_batch_run(hp3d_pm_ctx* ctx, const hp3d_view_desc* descs, int n,
         int meta[7] = {store, radius, stride, variant, persistent ? 1 : 0, chunk, counters};
         put(meta, sizeof meta);
         put(&ctx->batch_done.ptr, sizeof(void*));
+        // (the persistent kernel's list: its one launch holds its length and units)
+        const int list[2] = {persistent ? (int)plan.items.size() : 0, units};
+        put(list, sizeof list);
         put(plan.offset.data(), plan.offset.size() * sizeof(int));
         put(plan.count.data(), plan.count.size() * sizeof(int));
         put(plan.tiles.data(), plan.tiles.size() * sizeof(int));
