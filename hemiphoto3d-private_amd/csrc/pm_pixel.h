@@ -343,13 +343,14 @@ constexpr int kOutsideTaps = 4;   // taps a row from which source_cost tests win
 //
 // A row's neighbouring taps read the same cache lines, 64 a gather where the
 // hypotheses are random, and the L1 holds four gathers' worth: the row's gathers
-// have to come back to back, before other waves' push those lines out.  The
-// compiler does that by itself but in the masked loop of 11 FP32 quads (kBurst),
-// where it put 13 instructions of address arithmetic between any two: initial
-// cost, 11 x 11 taps, 2400x1800, 6 sources, 3.80 ms, against 3.01 with all
-// addresses first (with 3 waves to a SIMD instead of 4, 3.49 and 3.01);
-// 3200x2400, 3 sources, 3.30 and 2.79; 1600x1200, 4 sources, 0.93 and 0.86.
-template <int NT, int ST, int STORE, bool MASKED, bool ZCHK, int C>
+// have to come back to back, before other waves' push those lines out.  In the
+// initial cost the compiler does that by itself, but in the masked loop of 11 FP32
+// quads it put 13 instructions of address arithmetic between any two.  BURST forms
+// all addresses first: 11 x 11 taps, 2400x1800, 6 sources, 3.80 -> 3.01 ms (with 3
+// waves to a SIMD instead of 4, 3.49 and 3.01); 3200x2400, 3 sources, 3.30 -> 2.79;
+// 1600x1200, 4 sources, 0.93 -> 0.86.  (The persistent kernel's START, with 3 waves
+// and nothing sorted, lost 8 % by it.)
+template <int NT, int ST, int STORE, bool MASKED, bool ZCHK, int C, bool BURST>
 __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
                                            const float* __restrict__ lwin, int lp, float cx,
                                            float cy, float cz, float h00, float h01, float h10,
@@ -373,7 +374,7 @@ __device__ __forceinline__ void tap_window(const SrcImage<STORE>& img,
         const float* lrow = lwin + j * ST * lp;
 #pragma unroll
         for (int i0 = 0; i0 < NT; i0 += C) {
-            constexpr bool kBurst = MASKED && C >= 11 && STORE == kStoreF32;
+            constexpr bool kBurst = MASKED && BURST;
             static_assert(!kBurst || C == NT, "whole rows");
             typename SrcImage<STORE>::Quad q[C];
             unsigned idx[C];
@@ -568,7 +569,7 @@ __device__ __forceinline__ bool cand_plane(const DevView& v, int x, int y, doubl
 }
 
 // Cost 1 - NCC of one candidate plane against source s.
-template <int NT, int ST, int STORE, int C>
+template <int NT, int ST, int STORE, int C, bool BURST = false>
 __device__ __forceinline__ float source_cost(const DevView& v, int s,
                                              const float* __restrict__ lwin, int lp,
                                              const WinRef& wr, int x, int y, const CandPlane& g)
@@ -643,13 +644,13 @@ __device__ __forceinline__ float source_cost(const DevView& v, int s,
         if (__all(outside)) return 2.0f;
     }
     if (__all(inside)) {
-        tap_window<NT, ST, STORE, false, true, C>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
+        tap_window<NT, ST, STORE, false, true, C, BURST>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
                                                    t11, h20, h21, umax, vmax, wr, m, bu, bv);
     } else if (kZClear && __all(z_clear(cz, h20, h21, (float)R))) {
-        tap_window<NT, ST, STORE, true, false, C>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
+        tap_window<NT, ST, STORE, true, false, C, BURST>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
                                                    t11, h20, h21, umax, vmax, wr, m, bu, bv);
     } else {
-        tap_window<NT, ST, STORE, true, true, C>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
+        tap_window<NT, ST, STORE, true, true, C, BURST>(img, lwin, lp, tx, ty, cz, t00, t01, t10,
                                                   t11, h20, h21, umax, vmax, wr, m, bu, bv);
     }
     const int cnt = m.cnt;
@@ -719,7 +720,7 @@ struct TopCosts {
     }
 };
 
-template <int NT, int ST, int STORE, int C>
+template <int NT, int ST, int STORE, int C, bool BURST = false>
 __device__ __forceinline__ float cand_cost(const DevView& v, const float* __restrict__ lwin,
                                            int lp, const WinRef& wr, int x, int y, double rx,
                                            double ry, double rz, float d, float nx, float ny,
@@ -730,7 +731,7 @@ __device__ __forceinline__ float cand_cost(const DevView& v, const float* __rest
     TopCosts t;
     const bool small_k = v.top_k <= 3;   // wave-uniform
     for (int s = 0; s < v.S; ++s)
-        t.insert(source_cost<NT, ST, STORE, C>(v, s, lwin, lp, wr, x, y, g), small_k);
+        t.insert(source_cost<NT, ST, STORE, C, BURST>(v, s, lwin, lp, wr, x, y, g), small_k);
     return t.mean(v);
 }
 
@@ -924,8 +925,8 @@ __device__ __forceinline__ void cost_tile_sorted(const DevView& v, const float* 
         double rx, ry, rz;
         ray_fp64(v.kinv_d, x_o, y_o, rx, ry, rz);
         IO::st1(v.cost[parity], y_o * v.Wc + i_o,
-                cand_cost<NT, ST, STORE, kCostChunk<NT>>(v, lwin, G::LP, wr, x_o, y_o, rx, ry, rz,
-                                                         hh.x, hh.y, hh.z, hh.w));
+                cand_cost<NT, ST, STORE, kCostChunk<NT>, (NT >= 11 && STORE == kStoreF32)>(
+                    v, lwin, G::LP, wr, x_o, y_o, rx, ry, rz, hh.x, hh.y, hh.z, hh.w));
     }
 }
 
