@@ -323,6 +323,8 @@ hipError_t HostLink::drain(hipStream_t st)
 
 hipError_t HostLink::upload(const Seg* segs, size_t n, hipStream_t st)
 {
+    if (n == 1 && segs->bytes < kLoneUpload)
+        return hipMemcpyAsync(segs->dev, segs->host, segs->bytes, hipMemcpyHostToDevice, st);
     try {
         return through_ring(segs, n, false, st);
     } catch (const std::bad_alloc&) {

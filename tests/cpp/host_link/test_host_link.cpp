@@ -34,7 +34,13 @@ static bool both_ways(HostLink& link, hipStream_t st, size_t n)
 {
     const Bytes src = noise(n);
     Bytes dev(n), dst(n + 2);
-    CHECK(link.upload({{const_cast<unsigned char*>(src.data()), dev.data(), n}}, st) == hipSuccess);
+    const size_t half = n / 2;
+    unsigned char* from = const_cast<unsigned char*>(src.data());
+    CHECK(link.upload({{from, dev.data(), half}, {from + half, dev.data() + half, n - half}}, st) == hipSuccess);
+    CHECK(hipStreamSynchronize(st) == hipSuccess);
+    CHECK(dev == src);
+    std::fill(dev.begin(), dev.end(), 0);
+    CHECK(link.upload({{from, dev.data(), n}}, st) == hipSuccess);
     CHECK(hipStreamSynchronize(st) == hipSuccess);
     CHECK(dev == src);
     CHECK(link.download({{dst.data() + 1, dev.data(), n}}, st) == hipSuccess);
@@ -55,6 +61,28 @@ static bool sizes()
     for (size_t n : {(size_t)1, (size_t)63, (size_t)257}) CHECK(both_ways(link, &st, n));
     link.close();
     return both_ways(link, &st, 5 * M + 3);   // opened again
+}
+
+// One segment below 24 MiB goes up by the runtime's copy, without the ring; from there
+// on, and two segments, through it.
+static bool lone()
+{
+    HostLink link;
+    StubStream st;
+    const size_t line = 24u << 20;
+    Bytes src = noise(line), dev(line);
+    const auto up = [&](size_t a, size_t b) {
+        std::fill(dev.begin(), dev.end(), 0);
+        stub().pinned_copies = stub().pageable_copies = 0;
+        const HostLink::Seg segs[] = {{src.data(), dev.data(), a}, {src.data() + a, dev.data() + a, b}};
+        return link.upload(segs, b ? 2 : 1, &st) == hipSuccess && hipStreamSynchronize(&st) == hipSuccess &&
+               std::memcmp(dev.data(), src.data(), a + b) == 0;
+    };
+    CHECK(up(1, 0) && stub().pageable_copies == 1 && stub().pinned_copies == 0);
+    CHECK(up(line - 1, 0) && stub().pageable_copies == 1 && stub().pinned_copies == 0);
+    CHECK(up(line, 0) && stub().pageable_copies == 0 && stub().pinned_copies == 6);
+    CHECK(up(100, 200) && stub().pageable_copies == 0 && stub().pinned_copies == 1);
+    return true;
 }
 
 // Many odd segments, adjacent on the device or not, more of them to a piece than it has
@@ -131,12 +159,13 @@ static bool no_heap()
     HostLink bare;   // no ring, no threads, no lists yet
     for (HostLink* l : {&link, &bare}) {
         for (size_t upto = 0; upto < 2; ++upto) {
-            const HostLink::Seg up[] = {{const_cast<unsigned char*>(src.data()), dev.data(), n}};
+            unsigned char* from = const_cast<unsigned char*>(src.data());
+            const HostLink::Seg up[] = {{from, dev.data(), 1}, {from + 1, dev.data() + 1, n - 1}};
             const HostLink::Seg down[] = {{a.data(), dev.data(), n / 2},
                                           {b.data(), dev.data() + n / 2, n - n / 2}};
             std::fill(a.begin(), a.end(), 0);
             refuse_new = true;
-            const bool ok = l->upload(up, 1, &st) == hipSuccess && l->download(down, 2, &st) == hipSuccess;
+            const bool ok = l->upload(up, 2, &st) == hipSuccess && l->download(down, 2, &st) == hipSuccess;
             refuse_new = false;
             CHECK(ok);
             CHECK(std::memcmp(a.data(), src.data(), n / 2) == 0);
@@ -188,7 +217,7 @@ static bool sleeps()
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
-    const bool ok = what == "sizes" ? sizes() : what == "parts" ? parts() : what == "no_ring" ? no_ring()
+    const bool ok = what == "sizes" ? sizes() : what == "parts" ? parts() : what == "lone" ? lone() : what == "no_ring" ? no_ring()
                     : what == "no_heap" ? no_heap()
                     : what == "sleeps" ? sleeps() : false;
     std::puts(ok ? "ok" : "failed");

@@ -22,7 +22,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["sizes", "parts", "no_ring", "no_heap", "sleeps"])
+@pytest.mark.parametrize("check", ["sizes", "lone", "parts", "no_ring", "no_heap", "sleeps"])
 def test_host_link(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
