@@ -29,11 +29,12 @@ size_t job_state_bytes(int W, int H, int want_outputs_mask)
     size_t n = align256(2 * plane * sizeof(float4)) + align256(2 * plane * sizeof(float)) +
                align256(2 * plane);
     const size_t px = (size_t)W * H * sizeof(float);
-    if (want_outputs_mask & 1) n += align256(px);       // depth
-    if (want_outputs_mask & 2) n += align256(3 * px);   // normal
-    if (want_outputs_mask & 4) n += align256(px);       // cost
-    if (want_outputs_mask & 8) n += align256(px);       // confidence
-    return n;
+    size_t out = 0;
+    if (want_outputs_mask & 1) out += px;       // depth
+    if (want_outputs_mask & 2) out += 3 * px;   // normal
+    if (want_outputs_mask & 4) out += px;       // cost
+    if (want_outputs_mask & 8) out += px;       // confidence
+    return n + align256(out);
 }
 
 void bind_job(DevJob& j, const hp3d_view_desc* d, const Image* ref, const Image* const* srcs,
@@ -56,10 +57,12 @@ void bind_job(DevJob& j, const hp3d_view_desc* d, const Image* ref, const Image*
     j.v.chg[0] = chg;
     j.v.chg[1] = chg + plane;
     const size_t px = (size_t)j.v.W * j.v.H * sizeof(float);
-    if (outputs_mask & 1) { j.out_depth = reinterpret_cast<float*>(p); p += align256(px); }
-    if (outputs_mask & 2) { j.out_normal = reinterpret_cast<float*>(p); p += align256(3 * px); }
-    if (outputs_mask & 4) { j.out_cost = reinterpret_cast<float*>(p); p += align256(px); }
-    if (outputs_mask & 8) { j.out_conf = reinterpret_cast<float*>(p); p += align256(px); }
+    // the outputs without gaps: a small view's maps come over in one copy (an event
+    // and 10 us each otherwise)
+    if (outputs_mask & 1) { j.out_depth = reinterpret_cast<float*>(p); p += px; }
+    if (outputs_mask & 2) { j.out_normal = reinterpret_cast<float*>(p); p += 3 * px; }
+    if (outputs_mask & 4) { j.out_cost = reinterpret_cast<float*>(p); p += px; }
+    if (outputs_mask & 8) { j.out_conf = reinterpret_cast<float*>(p); p += px; }
     j.seed = d->seed;
 }
 
