@@ -85,8 +85,8 @@ __device__ __forceinline__ bool geom_consistent(const GeomViewDev& g, int x, int
 }
 
 // One 64x4-pixel tile per workgroup, tiles in XCD order: the source maps'
-// rows that a band of the view projects to stay in one XCD's L2.  Bound by
-// memory (37 us for a 1280x960 view with 8 sources, 4.3 TB/s).  kept[tile]:
+// rows that a band of the view projects to stay in one XCD's L2.  Bound by its
+// gathers (44 us for a 1280x960 view with 8 sources, 3.6 TB/s).  kept[tile]:
 // pixels left with a depth, which a pass over the downloaded maps on the host
 // took 1.1 ms to count for nine such views (null: not counted).
 __global__ __launch_bounds__(256) void geom_filter_kernel(GeomViewDev g, int tiles_x, int tiles,
