@@ -244,13 +244,14 @@ void HostLink::end()
     cv_.wait(lk, [&] { return inside_ == 0; });
 }
 
-// The copy out of the slot, over on return.  While copies follow each other that takes
-// tens of microseconds; where it takes longer, the stream is still at the work before
-// them (an earlier view's passes), and the threads sleep until it has come.
-hipError_t HostLink::slot_ready(int slot)
+// The copy out of the slot, over on return.  While copies follow each other (flowing)
+// that takes tens of microseconds; where it takes longer, the stream is still at the
+// work before them (an earlier view's passes), and the threads sleep until it has come.
+hipError_t HostLink::slot_ready(int slot, bool flowing)
 {
     if (!in_flight_[slot]) return hipSuccess;
     in_flight_[slot] = false;
+    if (flowing) return hipEventSynchronize(ev_[slot]);
     const auto patience = std::chrono::steady_clock::now() + std::chrono::microseconds(kPatienceUs);
     hipError_t e;
     while ((e = hipEventQuery(ev_[slot])) == hipErrorNotReady) {
@@ -342,7 +343,8 @@ hipError_t HostLink::fill(hipStream_t st)
         // without threads a piece at a time, so that the link starts early
         const size_t ahead = active_.load(std::memory_order_relaxed) ? kSlots : 1;
         while (handed < n && handed < issued + ahead && e == hipSuccess) {
-            e = slot_ready((int)(handed % kSlots));
+            // (behind its first slot's copy the stream is at this call's)
+            e = slot_ready((int)(handed % kSlots), handed > kSlots);
             if (e == hipSuccess) hand_out(handed++);
         }
         if (e != hipSuccess) break;

@@ -100,7 +100,7 @@ private:
     void wake();
     void hand_out(size_t piece);
     void end();
-    hipError_t slot_ready(int slot);
+    hipError_t slot_ready(int slot, bool flowing = false);
     char* slot_ptr(size_t piece) { return ring_ + (piece % kSlots) * kSlotBytes; }
 
     char* ring_ = nullptr;
